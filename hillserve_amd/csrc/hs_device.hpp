@@ -96,6 +96,13 @@ __device__ __forceinline__ bool finite_half(uint32_t bits) {
     return (bits & 0x7c00u) != 0x7c00u;
 }
 
+// 16-byte store past the caches' replacement order (the nontemporal hint):
+// for output that the launch does not read back.
+__device__ __forceinline__ void store_streaming(void* dst, uint4 v) {
+    typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+    __builtin_nontemporal_store(u32x4_t{v.x, v.y, v.z, v.w}, static_cast<u32x4_t*>(dst));
+}
+
 // Integer wave64 scans and reductions on DPP row moves, which stay in the
 // VALU (a __shfl is an LDS permute with its own round trip): row_shr 1, 2,
 // 4, 8 scan each row of 16 lanes; row_bcast:15 then adds row 0's total to
