@@ -1,9 +1,8 @@
 // Kernel #3 — physical union, packed-workspace build and row-map gather.
 //
-//  * hs_gqa_physical_union: runtime/gqa_pack.hpp:12-22.  One 32-bit
-//    membership word per visible id (bit h = query head h), duplicate and
-//    future ids rejected, then an order-preserving compaction of the nonzero
-//    words -> sorted unique ids.
+//  * hs_gqa_physical_union: runtime/gqa_pack.hpp:12-22.  One bitmap over the
+//    visible ids per query head, duplicate and future ids rejected, then an
+//    order-preserving compaction of their OR -> sorted unique ids.
 //  * hs_gqa_pack: runtime/gqa_pack.hpp:26-58, byte for byte: K
 //    [slot][Qhead][128], V transposed [Qhead][128][slot], mask
 //    [Qhead][qpad][slot] = 0 where id <= position[q], -inf elsewhere, zero
@@ -42,66 +41,112 @@ void launch_fill_u32(uint32_t* dst, uint32_t count, uint32_t value, hipStream_t 
 
 namespace {
 
-__device__ __forceinline__ void raise(hs_status_t* status, int code) {
-    atomicCAS(reinterpret_cast<int*>(&status->code), HS_OK, code);
-}
+// Physical union in two launches.  A head's list becomes a bitmap over the
+// visible ids in one workgroup's LDS (at most 66048 ids: 8.3 KB), where the
+// atomic's old word shows a duplicate, and is written out whole, so nothing
+// needs clearing first; the second launch ORs the 32 bitmaps and compacts.
+// Latency-bound: 32 x 6553 ids (0.8 MB in, 0.3 MB of bitmaps) take two
+// dependent launches of a few memory round trips each.  The five launches
+// before it (two fills, atomics on one global word per id, count, write)
+// took 13.4 us more at 32768 visible ids (union and pack 73.1 -> 59.7 us),
+// 6.1 us more at 8192 (23.8 -> 17.7 us) and 13.9 us more at 48001 (score,
+// cover and union 97.1 -> 83.2 us).
+constexpr uint32_t kUnionThreads = 1024;
+constexpr uint32_t kMaxUnionWords = (kMaxVisible + 31) / 32;  // 2064
+constexpr uint32_t kUnionBatch = 8;  // ids per thread requested before any is used
 
-__global__ void union_mark_kernel(const uint32_t* __restrict__ ids,
-                                  const uint32_t* __restrict__ lens, uint32_t ids_stride,
-                                  uint32_t visible, uint32_t* __restrict__ seen,
-                                  hs_status_t* __restrict__ status) {
-    const uint32_t h = blockIdx.y;
+// One workgroup per head: bitmap of its ids, and whether it holds a
+// duplicate or future id.
+__global__ void __launch_bounds__(kUnionThreads)
+union_mark_kernel(const uint32_t* __restrict__ ids, const uint32_t* __restrict__ lens,
+                  uint32_t ids_stride, uint32_t visible, uint32_t* __restrict__ bitmaps,
+                  uint32_t* __restrict__ bad_heads) {
+    __shared__ uint32_t bits[kMaxUnionWords];
+    __shared__ uint32_t bad;
+    const uint32_t h = blockIdx.x, tid = threadIdx.x, words = (visible + 31) / 32;
     const uint32_t len = lens[h];
-    for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < len;
-         j += gridDim.x * blockDim.x) {
-        const uint32_t id = ids[static_cast<size_t>(h) * ids_stride + j];
-        if (id >= visible) {
-            raise(status, HS_ERR_DUPLICATE);
-            continue;
+    const uint32_t* list = ids + static_cast<size_t>(h) * ids_stride;
+    for (uint32_t w = tid; w < words; w += kUnionThreads) bits[w] = 0;
+    if (tid == 0) bad = 0;
+    __syncthreads();
+    bool mine_bad = false;
+    for (uint64_t first = 0; first < len; first += kUnionThreads * kUnionBatch) {
+        uint32_t id[kUnionBatch];
+#pragma unroll
+        for (uint32_t u = 0; u < kUnionBatch; ++u) {  // (len >= 1 here: the index is clamped)
+            const uint64_t j = first + u * kUnionThreads + tid;
+            id[u] = list[j < len ? j : len - 1u];
         }
-        const uint32_t old = atomicOr(&seen[id], 1u << h);
-        if (old & (1u << h)) raise(status, HS_ERR_DUPLICATE);
+#pragma unroll
+        for (uint32_t u = 0; u < kUnionBatch; ++u) {
+            if (first + u * kUnionThreads + tid >= len) continue;
+            if (id[u] >= visible) {
+                mine_bad = true;
+                continue;
+            }
+            const uint32_t bit = 1u << (id[u] & 31u);
+            mine_bad |= (atomicOr(&bits[id[u] >> 5], bit) & bit) != 0;
+        }
     }
+    if (mine_bad) bad = 1;
+    __syncthreads();
+    for (uint32_t w = tid; w < words; w += kUnionThreads)
+        bitmaps[static_cast<size_t>(h) * words + w] = bits[w];
+    if (tid == 0) bad_heads[h] = bad;
 }
 
-// Per 1024-id block: number of ids seen by any head.
-__global__ void __launch_bounds__(1024)
-union_count_kernel(const uint32_t* __restrict__ seen, uint32_t visible,
-                   uint32_t* __restrict__ block_counts) {
-    __shared__ uint32_t tot[16];
-    const uint32_t i = blockIdx.x * 1024 + threadIdx.x;
-    const uint32_t v = (i < visible && seen[i]) ? 1u : 0u;
-    const uint32_t w = wave_sum_u32(v);
-    if ((threadIdx.x & 63u) == 0) tot[threadIdx.x >> 6] = w;
+// Workgroup b writes the union's ids of bitmap words 64 b .. 64 b + 63.  Its
+// place in the output is the number of union ids in the words before them,
+// which it counts itself from the bitmaps (at most 264 KB from L2), so the
+// workgroups wait for nothing.
+constexpr uint32_t kUnionWords = 64;
+__global__ void __launch_bounds__(kUnionThreads)
+union_write_kernel(const uint32_t* __restrict__ bitmaps, const uint32_t* __restrict__ bad_heads,
+                   uint32_t visible, uint32_t* __restrict__ out, uint32_t* __restrict__ out_n,
+                   hs_status_t* __restrict__ status) {
+    __shared__ uint32_t own[kUnionWords], first_at[kUnionWords];
+    __shared__ uint32_t before[kUnionThreads / 64];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, words = (visible + 31) / 32;
+    const uint32_t first = blockIdx.x * kUnionWords;
+    const uint32_t end = first + kUnionWords < words ? first + kUnionWords : words;
+    if (tid < kUnionWords) own[tid] = 0;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t s = 0;
-        for (uint32_t k = 0; k < 16; ++k) s += tot[k];
-        block_counts[blockIdx.x] = s;
+    uint32_t count = 0;
+    for (uint32_t w = tid; w < end; w += kUnionThreads) {
+        uint32_t v[32], any = 0;
+#pragma unroll
+        for (uint32_t h = 0; h < 32; ++h) v[h] = bitmaps[static_cast<size_t>(h) * words + w];
+#pragma unroll
+        for (uint32_t h = 0; h < 32; ++h) any |= v[h];
+        if (w < first) count += static_cast<uint32_t>(__popc(any));
+        else own[w - first] = any;
     }
-}
-
-__global__ void __launch_bounds__(1024)
-union_write_kernel(const uint32_t* __restrict__ seen, uint32_t visible,
-                   const uint32_t* __restrict__ block_counts, uint32_t blocks,
-                   uint32_t* __restrict__ out, uint32_t* __restrict__ out_n) {
-    __shared__ uint32_t tot[16];
-    __shared__ uint32_t offset;
-    if (threadIdx.x == 0) {
-        uint32_t s = 0;
-        for (uint32_t b = 0; b < blockIdx.x; ++b) s += block_counts[b];
-        offset = s;
-        if (blockIdx.x == blocks - 1) *out_n = s + block_counts[blockIdx.x];
-    }
-    const uint32_t i = blockIdx.x * 1024 + threadIdx.x;
-    const uint32_t v = (i < visible && seen[i]) ? 1u : 0u;
-    const uint64_t ballot = __ballot(v);
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    if (lane == 0) tot[wave] = static_cast<uint32_t>(__popcll(ballot));
+    count = wave_sum_u32(count);
+    if (lane == 0) before[tid >> 6] = count;
     __syncthreads();
-    uint32_t before = offset;
-    for (uint32_t k = 0; k < wave; ++k) before += tot[k];
-    if (v) out[before + lanes_below(ballot)] = i;
+    if (tid < kUnionWords) {  // wave 0
+        uint32_t at = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < kUnionThreads / 64; ++w) at += before[w];
+        const uint32_t c = static_cast<uint32_t>(__popc(own[tid]));
+        const uint32_t x = wave_inclusive_sum_u32(c);
+        first_at[tid] = at + x - c;
+        if (blockIdx.x == gridDim.x - 1 && tid == kUnionWords - 1) *out_n = at + x;
+        if (blockIdx.x == 0) {
+            const uint64_t any_bad = __ballot(tid < 32 && bad_heads[tid & 31u] != 0);
+            if (tid == 0) {
+                hs_status_t st{};
+                st.code = any_bad ? HS_ERR_DUPLICATE : HS_OK;
+                *status = st;
+            }
+        }
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i < kUnionWords * 32; i += kUnionThreads) {
+        const uint32_t w = i >> 5, b = i & 31u, x = own[w];
+        if ((x >> b) & 1u)
+            out[first_at[w] + static_cast<uint32_t>(__popc(x & ((1u << b) - 1u)))] = first * 32 + i;
+    }
 }
 
 // Source of one (slot, head) pair of the packed layout.
@@ -301,7 +346,7 @@ extern "C" {
 
 size_t hs_gqa_union_workspace_bytes(uint32_t visible) {
     const size_t v = visible ? visible : 1;
-    return hs::align256(v * 4) + hs::align256(((v + 1023) / 1024) * 4);
+    return hs::align256((v + 31) / 32 * 32 * 4) + hs::align256(32 * 4);
 }
 
 int hs_gqa_physical_union(const uint32_t* ids_dev, const uint32_t* lens_dev, size_t ids_stride,
@@ -313,20 +358,15 @@ int hs_gqa_physical_union(const uint32_t* ids_dev, const uint32_t* lens_dev, siz
     if (visible == 0 || visible > hs::kMaxVisible) return hs::reject("GQA union bounds");
     if (ids_stride > 0xffffffffu) return hs::reject("GQA union: ids_stride too large");
     hipStream_t s = hs::as_stream(stream);
-    uint32_t* seen = static_cast<uint32_t*>(workspace_dev);
-    const uint32_t blocks = (visible + 1023) / 1024;
-    uint32_t* block_counts =
-        reinterpret_cast<uint32_t*>(static_cast<char*>(workspace_dev) + hs::align256(size_t(visible) * 4));
-    hipLaunchKernelGGL(hs::fill_u32_kernel, dim3((visible + 255) / 256), dim3(256), 0, s, seen,
-                       visible, 0u);
-    hipLaunchKernelGGL(hs::fill_u32_kernel, dim3(1), dim3(256), 0, s,
-                       reinterpret_cast<uint32_t*>(status_dev), 4u, 0u);
-    hipLaunchKernelGGL(hs::union_mark_kernel, dim3(8, 32), dim3(256), 0, s, ids_dev, lens_dev,
-                       static_cast<uint32_t>(ids_stride), visible, seen, status_dev);
-    hipLaunchKernelGGL(hs::union_count_kernel, dim3(blocks), dim3(1024), 0, s, seen, visible,
-                       block_counts);
-    hipLaunchKernelGGL(hs::union_write_kernel, dim3(blocks), dim3(1024), 0, s, seen, visible,
-                       block_counts, blocks, out_dev, out_n_dev);
+    const uint32_t words = (visible + 31) / 32;
+    uint32_t* bitmaps = static_cast<uint32_t*>(workspace_dev);  // [32][words]
+    uint32_t* bad_heads = reinterpret_cast<uint32_t*>(static_cast<char*>(workspace_dev) +
+                                                      hs::align256(size_t(words) * 32 * 4));
+    hipLaunchKernelGGL(hs::union_mark_kernel, dim3(32), dim3(hs::kUnionThreads), 0, s, ids_dev,
+                       lens_dev, static_cast<uint32_t>(ids_stride), visible, bitmaps, bad_heads);
+    hipLaunchKernelGGL(hs::union_write_kernel, dim3((words + hs::kUnionWords - 1) / hs::kUnionWords),
+                       dim3(hs::kUnionThreads), 0, s, bitmaps, bad_heads, visible, out_dev,
+                       out_n_dev, status_dev);
     const hipError_t st = hipGetLastError();
     return st == hipSuccess ? HS_OK : hs::hip_fail(st, "union launch");
 }

@@ -185,3 +185,28 @@ def test_status_needs_no_clearing(hs, port):
     row_map[5] = 3  # beyond the two prefetched rows
     _, _, st = hs.ops.gather_rows(pre, None, to_dev(row_map), 32, status=status)
     assert hs.ops.read_status(st)["code"] == hs.HS_ERR_MISSING
+
+
+@pytest.mark.parametrize("visible", [1, 31, 32, 33, 2047, 2048, 2049, 66048])
+def test_union_bitmap_edges(hs, visible):
+    # ends of bitmap words, of a workgroup's 64 words and of the largest
+    # range; empty lists; then a duplicate and a future id in one head each
+    g = rng(70 + visible)
+    k = min(visible, 9000)  # more than one batch of 8192 ids of a head's workgroup
+    selected = [np.zeros(0, dtype=np.int64) for _ in range(32)]
+    for h in range(0, 32, 3):
+        selected[h] = g.choice(visible, size=int(g.integers(1, k + 1)), replace=False)
+    selected[30][0] = visible - 1 if visible - 1 not in selected[30] else selected[30][0]
+    ids, lens, stride = dev_ids(selected)
+    out, out_n, status = hs.ops.physical_union(ids, lens, stride, visible)
+    want = np.unique(np.concatenate(selected))
+    assert hs.ops.read_status(status) == {"code": 0, "k": 0, "boundary_tied_heads": 0, "head0_max_key": 0}
+    assert int(out_n.item()) == len(want)
+    assert np.array_equal(from_dev(out)[: len(want)], want.astype(np.uint32))
+    for extra in (int(selected[30][-1]), visible):
+        bad = [list(r) for r in selected]
+        bad[30].append(extra)
+        ids, lens, stride = dev_ids(bad)
+        out, out_n, status = hs.ops.physical_union(ids, lens, stride, visible)
+        assert hs.ops.read_status(status)["code"] == hs.HS_ERR_DUPLICATE
+        assert int(out_n.item()) == len(want)  # the refused id adds nothing
