@@ -32,9 +32,11 @@ struct CombineLds {
     float red[8];
     float acc16[kCombineRows][33];
 };
-__device__ __forceinline__ void combine_records(const float* __restrict__ part, uint32_t chunks,
-                                                float* __restrict__ out, uint32_t h,
-                                                uint32_t channel_group, CombineLds& lds) {
+// kFirst: o values per thread, at least ceil(chunks / kCombineRows).
+template <uint32_t kFirst>
+__device__ __forceinline__ void combine_batch(const float* __restrict__ part, uint32_t chunks,
+                                              float* __restrict__ out, uint32_t h,
+                                              uint32_t channel_group, CombineLds& lds) {
     auto& weight = lds.weight;
     auto& red = lds.red;
     auto& acc16 = lds.acc16;
@@ -43,7 +45,6 @@ __device__ __forceinline__ void combine_records(const float* __restrict__ part, 
     const float* recs = part + static_cast<size_t>(g) * chunks * 4 * kAttnRecord + j * kAttnRecord;
     const uint32_t c = tid & 31u, r = tid >> 5, ch = channel_group * 32 + c;
     const uint32_t last = chunks - 1;  // reads past the last chunk are clamped to it
-    constexpr uint32_t kFirst = 16;    // o values per thread in the first batch
     float v[kFirst];
 #pragma unroll
     for (uint32_t u = 0; u < kFirst; ++u)
@@ -68,7 +69,7 @@ __device__ __forceinline__ void combine_records(const float* __restrict__ part, 
     float L = 0.0f;
 #pragma unroll
     for (uint32_t w = 0; w < 8; ++w) L += red[w];
-    // the 16 weights are read before any is used (a read inside the test
+    // the weights are read before any is used (a read inside the test
     // below would make each term wait for its own LDS round trip); a zero
     // weight still skips its term, whose o may be inf or NaN
     float wv[kFirst];
@@ -79,10 +80,6 @@ __device__ __forceinline__ void combine_records(const float* __restrict__ part, 
     for (uint32_t u = 0; u < kFirst; ++u) {
         const uint32_t i = r + kCombineRows * u;
         if (i < chunks && wv[u] != 0.0f) a = __builtin_fmaf(v[u], wv[u], a);
-    }
-    for (uint32_t i = r + kCombineRows * kFirst; i < chunks; i += kCombineRows) {  // n > 32768
-        const float x = recs[i * 4 * kAttnRecord + 2 + ch];
-        if (weight[i] != 0.0f) a = __builtin_fmaf(x, weight[i], a);
     }
     acc16[r][c] = a;
     __syncthreads();
@@ -96,5 +93,23 @@ __device__ __forceinline__ void combine_records(const float* __restrict__ part, 
     }
 }
 
+// The batch is chosen by the number of chunks: 4, 16 or 32 values per thread
+// for n <= 8192, 32768 and 65536 (the order of the sum does not depend on
+// it).  A batch whose later values were read one by
+// one in a loop made n = 65536 wait a round trip per 16 chunks: its layer
+// takes 72.8 us with 32 values at once against 77.6.  The short batch takes
+// 28.0 against 28.3 us at n = 1024 and 28.4 against 29.0 at 4096, where most
+// of 16 values are the last chunk's again.
+__device__ __forceinline__ void combine_records(const float* __restrict__ part, uint32_t chunks,
+                                                float* __restrict__ out, uint32_t h,
+                                                uint32_t channel_group, CombineLds& lds) {
+    static_assert(kMaxChunks <= 32 * kCombineRows, "the widest batch covers every chunk");
+    if (chunks <= 4 * kCombineRows)
+        combine_batch<4>(part, chunks, out, h, channel_group, lds);
+    else if (chunks <= 16 * kCombineRows)
+        combine_batch<16>(part, chunks, out, h, channel_group, lds);
+    else
+        combine_batch<32>(part, chunks, out, h, channel_group, lds);
+}
 
 }  // namespace hs

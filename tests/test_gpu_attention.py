@@ -174,3 +174,19 @@ def test_closed_forms(hs, port, form, case):
     # (KV head 0's marker output is exactly zero: compare element-wise)
     ref = port.attention(q, pool_rows(k, v).view(np.uint8), [list(r) for r in ids])
     assert np.allclose(got, ref, rtol=TOL, atol=1e-5)
+
+
+@pytest.mark.parametrize("n", [128 * 64, 128 * 64 + 1, 28671, 28672, 128 * 256 + 1, 65536])
+def test_merge_batches_and_streamed_rows(hs, port, n):
+    # the record merge reads 4, 16 or 32 chunks per thread (64, 256 and 512
+    # chunks of 128 ids), and the V rows are streamed from 28672 tokens on
+    g = rng(50 + n)
+    k = f16_bits(g.standard_normal((n, 8, 128)))
+    v = f16_bits(g.standard_normal((n, 8, 128)))
+    pool = pool_rows(k, v)
+    q = g.standard_normal((32, 128)).astype(np.float32)
+    ids = [np.unique(np.append(g.choice(n, size=n // 100, replace=False), n - 1)) for _ in range(32)]
+    out = hs.ops.sparse_attention(torch.from_numpy(q).cuda(), to_dev(pool.reshape(-1)), n,
+                                  to_dev(member_words(ids, n).reshape(-1)))
+    ref = port.attention(q, pool.view(np.uint8), ids)
+    assert rel_err(out.cpu().numpy().astype(np.float64), ref) <= TOL
