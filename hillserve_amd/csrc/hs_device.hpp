@@ -96,6 +96,13 @@ __device__ __forceinline__ bool finite_half(uint32_t bits) {
     return (bits & 0x7c00u) != 0x7c00u;
 }
 
+// 16-byte load with the nontemporal hint: for data that nothing reads again
+// before it would have left the caches anyway.
+__device__ __forceinline__ uint4 load_streaming(const void* src) {
+    typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+    const u32x4_t x = __builtin_nontemporal_load(static_cast<const u32x4_t*>(src));
+    return make_uint4(x.x, x.y, x.z, x.w);
+}
 // 16-byte store past the caches' replacement order (the nontemporal hint):
 // for output that the launch does not read back.
 __device__ __forceinline__ void store_streaming(void* dst, uint4 v) {

@@ -40,26 +40,42 @@ namespace {
 
 constexpr uint32_t kWavesPerBlock = 2;
 
-template <bool kRows, bool kBatch>
+// Keys are streamed past the caches (nontemporal loads) where nothing will
+// read them again while the 256 MB MALL still holds them: they then stop
+// displacing the scores and dots that the next launches read, and a long
+// stream runs faster.  The dots' launch leaves the attention only V
+// rows to read, so its keys are done with: streamed from 56 MiB (28672
+// tokens), where the pools of a few layers no longer fit the MALL together.
+// One layer 46.0 -> 43.7 us at 32768 tokens, 73.5 -> 67.7 at 65536; below the
+// line it would lose what the MALL holds from the pass before (24576 tokens
+// 39.5 -> 41.3 us, 16384 33.2 -> 35.2).  A plain scoring launch is followed
+// by an attention that reads the selected K rows, so its line is 128 MiB,
+// more than the MALL keeps until then: 16 sequences of 8192 to 32768 tokens
+// 173.8 -> 155.8 us, a 65536-token cover 81.7 -> 77.4 us, while the pipelined
+// 32768-token layers (64 MiB a launch) would lose 2.4 us each.
+constexpr uint64_t kStreamKeyBytes = uint64_t(128) << 20;
+constexpr uint64_t kStreamLogitKeyBytes = uint64_t(56) << 20;
+
+template <bool kRows, bool kBatch, bool kStream>
 __global__ void __launch_bounds__(kWavesPerBlock * 64)
 score_kernel(const ScoreJobs jobs, const int32_t* __restrict__ rows, uint32_t pool_rows) {
     __shared__ uint4 lds[kWavesPerBlock][kHalfTileChunks];
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    score_waves<kRows, kBatch>(jobs, rows, pool_rows,
-                               __builtin_amdgcn_readfirstlane(blockIdx.x * kWavesPerBlock + w),
-                               gridDim.x * kWavesPerBlock, lds[w]);
+    score_waves<kRows, kBatch, false, kStream>(
+        jobs, rows, pool_rows, __builtin_amdgcn_readfirstlane(blockIdx.x * kWavesPerBlock + w),
+        gridDim.x * kWavesPerBlock, lds[w]);
 }
 
 // The scorer with the attention dots in the same pass (one job): each wave
 // also holds its KV head's split query (2 KiB of LDS); one half ahead.
-template <bool kRows>
+template <bool kRows, bool kStream>
 __global__ void __launch_bounds__(kWavesPerBlock * 64) __attribute__((amdgpu_waves_per_eu(4)))
 score_logits_kernel(const ScoreJobs jobs, const int32_t* __restrict__ rows, uint32_t pool_rows,
                     const LogitsOut lo) {
     __shared__ uint4 lds[kWavesPerBlock][kHalfTileChunks];
     __shared__ uint4 qstage[kWavesPerBlock][8 * 16];
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    score_waves<kRows, false, true>(
+    score_waves<kRows, false, true, kStream>(
         jobs, rows, pool_rows, __builtin_amdgcn_readfirstlane(blockIdx.x * kWavesPerBlock + w),
         gridDim.x * kWavesPerBlock, lds[w], lo, qstage[w]);
 }
@@ -102,15 +118,17 @@ int launch_score(const uint16_t* q, const uint16_t* keys, size_t stride_words,
     const LogitsOut lo{qf, logits, static_cast<uint32_t>(logit_stride), vec};
     jobs.total_ids = ((tokens + kTileTokens - 1) / kTileTokens) * 8;  // (token tile, KV head)
     const dim3 grid(score_grid(jobs.total_ids)), block(kWavesPerBlock * 64);
-    if (logits && rows)
-        hipLaunchKernelGGL(score_logits_kernel<true>, grid, block, 0, stream, jobs, rows, pool_rows,
-                           lo);
-    else if (logits)
-        hipLaunchKernelGGL(score_logits_kernel<false>, grid, block, 0, stream, jobs, rows, 0u, lo);
-    else if (rows)
-        hipLaunchKernelGGL((score_kernel<true, false>), grid, block, 0, stream, jobs, rows, pool_rows);
-    else
-        hipLaunchKernelGGL((score_kernel<false, false>), grid, block, 0, stream, jobs, rows, 0u);
+    const uint64_t key_bytes = uint64_t(tokens) * 2048;
+    const bool streamed = key_bytes >= (logits ? kStreamLogitKeyBytes : kStreamKeyBytes);
+    if (logits) {
+        const auto kernel = rows ? (streamed ? score_logits_kernel<true, true> : score_logits_kernel<true, false>)
+                                 : (streamed ? score_logits_kernel<false, true> : score_logits_kernel<false, false>);
+        hipLaunchKernelGGL(kernel, grid, block, 0, stream, jobs, rows, rows ? pool_rows : 0u, lo);
+    } else {
+        const auto kernel = rows ? (streamed ? score_kernel<true, false, true> : score_kernel<true, false, false>)
+                                 : (streamed ? score_kernel<false, false, true> : score_kernel<false, false, false>);
+        hipLaunchKernelGGL(kernel, grid, block, 0, stream, jobs, rows, rows ? pool_rows : 0u);
+    }
     const hipError_t status = hipGetLastError();
     return status == hipSuccess ? HS_OK : hip_fail(status, "score launch");
 }
@@ -142,8 +160,12 @@ int launch_score_batched(const hs_score_job_t* jobs, uint32_t count, hipStream_t
     ScoreJobs table;
     const int rc = build_score_jobs(jobs, count, table);
     if (rc != HS_OK) return rc;
-    hipLaunchKernelGGL((score_kernel<false, true>), dim3(score_grid(table.total_ids)),
-                       dim3(kWavesPerBlock * 64), 0, stream, table, nullptr, 0u);
+    uint64_t key_bytes = 0;
+    for (uint32_t i = 0; i < count; ++i) key_bytes += uint64_t(jobs[i].tokens) * 2048;
+    const auto kernel = key_bytes >= kStreamKeyBytes ? score_kernel<false, true, true>
+                                                     : score_kernel<false, true, false>;
+    hipLaunchKernelGGL(kernel, dim3(score_grid(table.total_ids)), dim3(kWavesPerBlock * 64), 0,
+                       stream, table, nullptr, 0u);
     const hipError_t status = hipGetLastError();
     return status == hipSuccess ? HS_OK : hip_fail(status, "score batch launch");
 }

@@ -65,7 +65,9 @@ int build_score_jobs(const hs_score_job_t* jobs, uint32_t count, ScoreJobs& out)
 // of LDS per wave), staged when the KV head changes.  Lane 4b + j ends with
 // head j's dots of tokens 4b .. 4b+3, written to lo.out unscaled; the
 // attention then reads V rows only.
-template <bool kRows, bool kBatch, bool kLogits = false>
+// kStream: the keys are read with the nontemporal hint (the launches decide,
+// score.hip).
+template <bool kRows, bool kBatch, bool kLogits = false, bool kStream = false>
 __device__ __forceinline__ void score_waves(const ScoreJobs& jobs, const int32_t* __restrict__ rows,
                                             uint32_t pool_rows, uint32_t wave, uint32_t waves,
                                             uint4* region, const LogitsOut& lo = LogitsOut{},
@@ -105,8 +107,8 @@ __device__ __forceinline__ void score_waves(const ScoreJobs& jobs, const int32_t
 #pragma unroll
         for (uint32_t j = 0; j < kHalf; ++j) {
             const bool ok = r[j] != 0xffffffffu;
-            const uint4 x = *reinterpret_cast<const uint4*>(
-                base + static_cast<size_t>(ok ? r[j] : 0u) * jb.stride_words);
+            const uint16_t* at = base + static_cast<size_t>(ok ? r[j] : 0u) * jb.stride_words;
+            const uint4 x = kStream ? load_streaming(at) : *reinterpret_cast<const uint4*>(at);
             v[j] = ok ? x : make_uint4(0u, 0u, 0u, 0u);
         }
     };

@@ -82,3 +82,26 @@ def test_attention_from_dots(hs, port, n, frac, mapped):
     via_k = hs.ops.sparse_attention(qd, k_rows, n, member, rows=rows, v_pool=v_rows,
                                     row_bytes=2048).cpu().numpy().astype(np.float64)
     assert rel_err(got, via_k) <= 1e-3
+
+
+@pytest.mark.parametrize("n", [28671, 28672, 65536])
+def test_streamed_keys(hs, n):
+    # keys are streamed from 28672 tokens in the dots' launch and from 65536
+    # in plain scoring (single and batched): the same bits as calls below
+    # those lines over parts of the keys
+    keys = torch.empty(n * 1024, dtype=torch.float16, device="cuda")
+    hs.ops.fill_rope_keys(keys, n, 1024, 8, seed=n)
+    q16 = torch.empty(4096, dtype=torch.float16, device="cuda")
+    hs.ops.fill_gaussian(q16, seed=n + 1)
+    q32 = torch.randn((32, 128), device="cuda")
+    raw, dots = hs.ops.score_logits(q16, q32, keys, n)
+    plain = hs.ops.score(q16, keys, n)
+    batch = hs.ops.score_batched([dict(q16=q16, keys=keys[a * 1024:], tokens=min(16384, n - a))
+                                  for a in range(0, n, 16384)])
+    for a, got in zip(range(0, n, 16384), batch):
+        part = keys[a * 1024:(a + 16384) * 1024]
+        tokens = part.numel() // 1024
+        want, want_dots = hs.ops.score_logits(q16, q32, part, tokens)
+        assert torch.equal(got, want)
+        assert torch.equal(raw[:, a:a + tokens], want) and torch.equal(plain[:, a:a + tokens], want)
+        assert torch.equal(dots[:, a:a + tokens], want_dots)
