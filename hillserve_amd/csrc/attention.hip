@@ -99,7 +99,13 @@ __device__ __forceinline__ void accumulate_pair(float (&o)[4][8], const half2v (
 //     l%16): 16 B of rows 16t + 4i + l/16);
 //  4. the chunk's exact maximum per head, p = exp(s - m) and l = sum p (no
 //     running maximum), then o += p * V as the rows land, and the record.
-template <bool kRows>
+// kStream: the V rows, which nothing reads again, are read with the
+// nontemporal hint, so that they leave the K rows (scored shortly before) in
+// the caches.  Eight pipelined layers of 32768 tokens take
+// 364.7 us against 368.0; no difference at 24576 and below, where the V rows
+// of a pass may come from the caches themselves.
+constexpr uint32_t kStreamTokens = 28672;
+template <bool kRows, bool kStream>
 __global__ void __launch_bounds__(kThreads)
 attn_kv_kernel(const float* __restrict__ q, const uint8_t* __restrict__ pool, uint32_t row_bytes,
                int64_t v_delta, const int32_t* __restrict__ rows, uint32_t pool_rows,
@@ -221,7 +227,8 @@ attn_kv_kernel(const float* __restrict__ q, const uint8_t* __restrict__ pool, ui
 #pragma unroll
             for (uint32_t i = 0; i < 4; ++i) {
                 const uint32_t r = 16 * t + 4 * i + q16 < total ? rr[i] : last_row;
-                vw[t][i] = *reinterpret_cast<const uint4*>(vbase + static_cast<size_t>(r) * row_bytes);
+                const uint8_t* at = vbase + static_cast<size_t>(r) * row_bytes;
+                vw[t][i] = kStream ? load_streaming(at) : *reinterpret_cast<const uint4*>(at);
             }
         }
     }
@@ -526,14 +533,12 @@ int launch_attention_partial(const float* q, const uint8_t* k_pool, const uint8_
     const int64_t v_delta = reinterpret_cast<intptr_t>(v_pool) - reinterpret_cast<intptr_t>(k_pool);
     const uint32_t chunks = (n + kChunk - 1) / kChunk;
     float* part = static_cast<float*>(workspace);
-    if (rows)
-        hipLaunchKernelGGL(attn_kv_kernel<true>, dim3(chunks), dim3(kThreads), 0, stream, q,
-                           k_pool, static_cast<uint32_t>(row_bytes), v_delta, rows, pool_rows,
-                           member, n, chunks, part);
-    else
-        hipLaunchKernelGGL(attn_kv_kernel<false>, dim3(chunks), dim3(kThreads), 0, stream,
-                           q, k_pool, static_cast<uint32_t>(row_bytes), v_delta, rows, 0u, member,
-                           n, chunks, part);
+    const bool streamed = n >= kStreamTokens;
+    const auto kernel = rows ? (streamed ? attn_kv_kernel<true, true> : attn_kv_kernel<true, false>)
+                             : (streamed ? attn_kv_kernel<false, true> : attn_kv_kernel<false, false>);
+    hipLaunchKernelGGL(kernel, dim3(chunks), dim3(kThreads), 0, stream, q, k_pool,
+                       static_cast<uint32_t>(row_bytes), v_delta, rows, rows ? pool_rows : 0u,
+                       member, n, chunks, part);
     const hipError_t st = hipGetLastError();
     return st == hipSuccess ? HS_OK : hip_fail(st, "attention launch");
 }
