@@ -18,16 +18,13 @@
 //                       coalesced 16 B reads into the device staging rows
 //                       (its K half to k_out + i * row_bytes, its V half to
 //                       v_out + i * row_bytes; the record layout itself is
-//                       (out, out + 2048, 4096)) and checks the header
-//                       identity;
-//   cold_digest_kernel: one lane per record hashes its staged K then V half
-//                       in byte order (FNV-1a is sequential within a record)
-//                       and compares the digest;
+//                       (out, out + 2048, 4096)), checks the header identity
+//                       and hashes the row from the same registers;
 //   cold_status_kernel: folds the per-record flags into the status.
 // hs_kv_cold_fetch_runs moves the same records over the host link with the
 // copy engines instead: one hipMemcpyAsync per run of consecutive positions
 // into a raw staging buffer in HBM (4128 B records, back to back), after
-// which the same three kernels check and split them there, so no CU waits
+// which the same kernels check and split them there, so no CU waits
 // on the host link.
 #include <hip/hip_runtime.h>
 
@@ -42,27 +39,98 @@ namespace hs {
 namespace {
 
 constexpr uint32_t kPad = 0xffffffffu;  // a position list's padding entry: no record
-constexpr uint32_t kPadFlag = 4u;
-// Workgroups (4 waves each) of a copy over the host link: 96 records of
-// 4 KiB in flight keep it at ~52 GB/s (16 workgroups: 50.5 GB/s, 8: 31)
-// while the CUs left free run the main stream's attention within 2x of its
-// speed alone (one wave per record over the whole chip: 7x).
-constexpr uint32_t kLinkBlocks = 24;
+constexpr uint32_t kPadFlag = 4u;  // a padding entry's flag; 1: a bad record
+// Waves of a copy over the host link: 96 records of 4 KiB in flight keep it
+// at ~56 GB/s, two waves on each of 48 CUs.  One sequence's fetch and
+// attention at 8192 tokens, half of them cold: 337 us; the same waves on 24
+// CUs 351, on 96 CUs 341, 128 waves on 32 / 64 CUs 345 / 368, 192 waves on 24
+// CUs 393 (more requests than the link takes queue up).  The CUs left free
+// run the main stream's attention within 2x of its speed alone (one wave per
+// record over the whole chip: 7x).
+constexpr uint32_t kLinkBlocks = 48;
+constexpr uint32_t kCopyThreads = 128, kCopyWaves = kCopyThreads / 64;
 
-// Record i (position positions[i]) into its staging row: copy, header identity.
+// FNV-1a 64 of a 4096 B row held by a wave, lane l with its 16 B words
+// l, 64 + l, 128 + l and 192 + l.  The hash h' = (h ^ b) p is sequential, but
+// only its low byte is more than linear: h ^ b = h + d where d depends on h's
+// low byte alone, and that byte's own chain, l' = (l ^ b) p mod 256, needs no
+// higher bit of h.  Bit k of l' is bit k of l, flipped by the bytes and the
+// bits below k.  So
+//  1. the low byte before every 16 B word is found one bit at a time: each
+//     lane runs its words' low-byte chains from the bits known so far, and the
+//     flips of bit k over the words before a word add up (parity) by ballot;
+//  2. every word is hashed from its low byte l alone, h(l); the true hash
+//     before it, h, adds (h - l) p^16, so the row's hash is the sum of
+//     (h(l) - l p^16) p^(16 words after it), plus the seed's seed p^4096.
+// About 1400 instructions per record, behind the copy's own waits, where one
+// lane of a launch of its own took 4096 dependent 64-bit multiplies over the
+// staged row: 53 us per fetch of 4096 records.  The fetch and attention at
+// 1024 tokens, half of them cold, take 74 us against 123, at 8192 337
+// against 388.
+constexpr uint64_t fnv_power(uint32_t e) {  // p^e mod 2^64
+    uint64_t r = 1, b = kFnvPrime;
+    for (; e != 0; e >>= 1, b *= b)
+        if (e & 1u) r *= b;
+    return r;
+}
+// p^(16 (63 - lane)): the weight of a lane's words within a block of 64
+__device__ __forceinline__ uint64_t lane_weight(uint32_t lane) {
+    constexpr uint64_t kPower[6] = {fnv_power(16), fnv_power(32), fnv_power(64),
+                                    fnv_power(128), fnv_power(256), fnv_power(512)};
+    uint64_t w = 1;
+#pragma unroll
+    for (uint32_t b = 0; b < 6; ++b) w *= ((63u - lane) >> b) & 1u ? kPower[b] : 1ull;
+    return w;
+}
+__device__ __forceinline__ uint64_t row_digest(const uint4 (&v)[4], uint32_t lane, uint64_t weight) {
+    uint32_t start[4] = {0u, 0u, 0u, 0u};  // the low byte before each word, bits known so far
+#pragma unroll 1
+    for (uint32_t bit = 0; bit < 8; ++bit) {
+        uint32_t flipped = static_cast<uint32_t>(kFnvSeed >> bit);  // bit 0: this bit so far
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            const uint32_t words[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
+            uint32_t l = start[j];
+#pragma unroll
+            for (uint32_t c = 0; c < 4; ++c)
+#pragma unroll
+                for (uint32_t b = 0; b < 4; ++b)  // (bits past the low byte never come back into it)
+                    l = __umul24(l ^ (words[c] >> (8 * b)), static_cast<uint32_t>(kFnvPrime & 0xffu));
+            const uint64_t flips = __ballot((l >> bit) & 1u);
+            start[j] |= ((flipped + lanes_below(flips)) & 1u) << bit;
+            flipped += static_cast<uint32_t>(__popcll(flips));
+        }
+    }
+    constexpr uint64_t kWord = fnv_power(16), kBlock = fnv_power(1024);
+    uint64_t sum = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+        const uint32_t words[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
+        uint64_t h = start[j];
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c)
+#pragma unroll
+            for (uint32_t b = 0; b < 4; ++b) h = (h ^ ((words[c] >> (8 * b)) & 0xffu)) * kFnvPrime;
+        sum = sum * kBlock + (h - start[j] * kWord);
+    }
+    sum *= weight;
+#pragma unroll
+    for (uint32_t off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+    return sum + kFnvSeed * fnv_power(4096);
+}
+
+// Record i (position positions[i]) into its staging row: copy, header
+// identity and digest; flags[i] != 0 marks a bad record or padding.
 template <bool kStaged>
 __device__ __forceinline__ void copy_record(const uint8_t* __restrict__ image, uint32_t layer,
                                             uint32_t capacity, uint64_t request,
                                             const uint32_t* __restrict__ positions, uint32_t i,
                                             uint8_t* k_out, uint32_t row_bytes, int64_t v_delta,
-                                            uint64_t* __restrict__ digests,
-                                            uint32_t* __restrict__ flags, uint32_t lane) {
+                                            uint32_t* __restrict__ flags, uint32_t lane,
+                                            uint64_t weight) {
     const uint32_t p = positions[i];
     if (p == kPad || p >= capacity) {  // padding entry, or nothing to read
-        if (lane == 0) {
-            flags[i] = p == kPad ? kPadFlag : 1u;
-            digests[i] = 0;
-        }
+        if (lane == 0) flags[i] = p == kPad ? kPadFlag : 1u;
         return;
     }
     const uint8_t* rec = kStaged ? image + uint64_t(i) * kStride
@@ -80,11 +148,11 @@ __device__ __forceinline__ void copy_record(const uint8_t* __restrict__ image, u
     // lane 0: digest, position; lane 1: request, layer | version << 32
     const uint64_t a = (uint64_t(hdr.y) << 32) | hdr.x, b = (uint64_t(hdr.w) << 32) | hdr.z;
     const uint64_t request_in = __shfl(a, 1, 64), ident = __shfl(b, 1, 64);
+    const uint64_t digest = row_digest(v, lane, weight);
     if (lane == 0) {
-        const bool ok = b == p && request_in == request && uint32_t(ident) == layer &&
+        const bool ok = a == digest && b == p && request_in == request && uint32_t(ident) == layer &&
                         uint32_t(ident >> 32) == 1u;
         flags[i] = ok ? 0u : 1u;
-        digests[i] = a;
     }
 }
 
@@ -96,53 +164,17 @@ __device__ __forceinline__ void copy_record(const uint8_t* __restrict__ image, u
 // staging buffer of hs_kv_cold_fetch_runs), expected at position
 // positions[i]; otherwise record (layer, positions[i]) of the image.
 template <bool kStaged>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(kCopyThreads)
 cold_copy_kernel(const uint8_t* __restrict__ image, uint32_t layer, uint32_t capacity,
                  uint64_t request, const uint32_t* __restrict__ positions, uint32_t count,
                  uint8_t* k_out, uint32_t row_bytes, int64_t v_delta,
-                 uint64_t* __restrict__ digests, uint32_t* __restrict__ flags) {
+                 uint32_t* __restrict__ flags) {
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t waves = gridDim.x * 4;
-    for (uint32_t i = blockIdx.x * 4 + (threadIdx.x >> 6); i < count; i += waves)
+    const uint32_t waves = gridDim.x * kCopyWaves;
+    const uint64_t weight = lane_weight(lane);
+    for (uint32_t i = blockIdx.x * kCopyWaves + (threadIdx.x >> 6); i < count; i += waves)
         copy_record<kStaged>(image, layer, capacity, request, positions, i, k_out, row_bytes,
-                             v_delta, digests, flags, lane);
-}
-
-// One lane per record: FNV-1a 64 over the staged row (K half, then V half),
-// in byte order.
-__global__ void __launch_bounds__(256)
-cold_digest_kernel(const uint8_t* k_rows, uint32_t row_bytes, int64_t v_delta,
-                   const uint64_t* __restrict__ digests, uint32_t count,
-                   uint32_t* __restrict__ flags) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= count || (flags[i] & kPadFlag)) return;
-    const uint8_t* k = k_rows + uint64_t(i) * row_bytes;
-    uint64_t h = kFnvSeed;
-    // 128 B per step, the next step's loads requested before this step's
-    // bytes are hashed (the hash chain is sequential; the loads need not be)
-    constexpr uint32_t kStep = 8;  // 16 B words per step
-    auto chunk = [&](uint32_t c) {
-        return reinterpret_cast<const uint4*>(k + (c < 128 ? 0 : v_delta - 2048) + c * 16);
-    };
-    uint4 cur[kStep], nxt[kStep];
-#pragma unroll
-    for (uint32_t u = 0; u < kStep; ++u) cur[u] = *chunk(u);
-    for (uint32_t c0 = 0; c0 < kRow / 16; c0 += kStep) {
-        const uint32_t c1 = c0 + kStep < kRow / 16 ? c0 + kStep : c0;  // last step re-reads its own
-#pragma unroll
-        for (uint32_t u = 0; u < kStep; ++u) nxt[u] = *chunk(c1 + u);
-#pragma unroll
-        for (uint32_t u = 0; u < kStep; ++u) {
-            const uint32_t words[4] = {cur[u].x, cur[u].y, cur[u].z, cur[u].w};
-#pragma unroll
-            for (uint32_t w = 0; w < 4; ++w)
-#pragma unroll
-                for (uint32_t b = 0; b < 4; ++b) h = (h ^ ((words[w] >> (8 * b)) & 0xffu)) * kFnvPrime;
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < kStep; ++u) cur[u] = nxt[u];
-    }
-    if (h != digests[i]) flags[i] |= 2u;
+                             v_delta, flags, lane, weight);
 }
 
 // Status: code HS_ERR_CORRUPT when any record failed, k = failed records.
@@ -164,7 +196,7 @@ cold_status_kernel(const uint32_t* __restrict__ flags, uint32_t count, hs_status
         }
 #pragma unroll
         for (uint32_t u = 0; u < kStatusBatch; ++u)
-            mine += base + threadIdx.x + u * kStatusThreads < count && (f[u] & 3u) ? 1u : 0u;
+            mine += base + threadIdx.x + u * kStatusThreads < count && (f[u] & 1u) ? 1u : 0u;
     }
     mine = wave_sum_u32(mine);
     if ((threadIdx.x & 63u) == 0 && mine) atomicAdd(&bad, mine);
@@ -271,8 +303,7 @@ cold_plan_kernel(const uint32_t* __restrict__ member, uint32_t heads, uint32_t n
 }  // namespace
 
 size_t cold_fetch_workspace_bytes(uint32_t count) {
-    const size_t n = count ? count : 1;
-    return align256(sizeof(uint64_t) * n) + align256(sizeof(uint32_t) * n);
+    return align256(sizeof(uint32_t) * (count ? count : 1));
 }
 
 // Host checks shared by both reads; the image header is host memory, so the
@@ -298,23 +329,20 @@ int check_cold_read(const void* image, uint32_t layer, const uint32_t* positions
 }
 
 // The check and split of `count` records (the copy kernel reads the image or
-// the staged records), the digest and the status.
+// the staged records) and the status.
 template <bool kStaged>
 int launch_cold_checks(const uint8_t* records, uint32_t layer, const uint64_t (&h)[8],
                        const uint32_t* positions, uint32_t count, uint8_t* k_out, uint8_t* v_out,
                        size_t row_bytes, hs_status_t* status, void* workspace, hipStream_t stream) {
     const int64_t v_delta = reinterpret_cast<intptr_t>(v_out) - reinterpret_cast<intptr_t>(k_out);
-    uint64_t* digests = static_cast<uint64_t*>(workspace);
-    uint32_t* flags = reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) +
-                                                  align256(sizeof(uint64_t) * count));
+    uint32_t* flags = static_cast<uint32_t*>(workspace);
     // over the host link a few workgroups keep the link busy (the copy is its
     // rate, not theirs); staged records in HBM take the whole chip
-    const uint32_t blocks = kStaged ? (count + 3) / 4 : std::min((count + 3) / 4, kLinkBlocks);
-    hipLaunchKernelGGL(cold_copy_kernel<kStaged>, dim3(blocks), dim3(256), 0, stream,
+    const uint32_t all = (count + kCopyWaves - 1) / kCopyWaves;
+    const uint32_t blocks = kStaged ? all : std::min(all, kLinkBlocks);
+    hipLaunchKernelGGL(cold_copy_kernel<kStaged>, dim3(blocks), dim3(kCopyThreads), 0, stream,
                        records, layer, static_cast<uint32_t>(h[4]), h[2], positions, count, k_out,
-                       static_cast<uint32_t>(row_bytes), v_delta, digests, flags);
-    hipLaunchKernelGGL(cold_digest_kernel, dim3((count + 255) / 256), dim3(256), 0, stream, k_out,
-                       static_cast<uint32_t>(row_bytes), v_delta, digests, count, flags);
+                       static_cast<uint32_t>(row_bytes), v_delta, flags);
     hipLaunchKernelGGL(cold_status_kernel, dim3(1), dim3(kStatusThreads), 0, stream, flags, count, status);
     const hipError_t st = hipGetLastError();
     return st == hipSuccess ? HS_OK : hip_fail(st, "cold fetch launch");

@@ -270,7 +270,7 @@ int hs_kv_store_append(void *image, uint32_t layer, uint32_t first, const uint8_
  * its output row is left as it was.  status_dev: code HS_ERR_CORRUPT and k
  * = number of bad records, else HS_OK.  The header page is read by the host
  * call.
- * workspace: hs_kv_cold_fetch_workspace_bytes(count).  3 launches. */
+ * workspace: hs_kv_cold_fetch_workspace_bytes(count).  2 launches. */
 size_t hs_kv_cold_fetch_workspace_bytes(uint32_t count);
 int hs_kv_cold_fetch(const void *image, uint32_t layer, const uint32_t *positions_dev,
                      uint32_t count, uint8_t *k_out_dev, uint8_t *v_out_dev, size_t row_bytes,

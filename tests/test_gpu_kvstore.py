@@ -199,3 +199,30 @@ def test_runs_fetch_corruption_and_rejections(hs):
                                      vp(out), ctypes.c_void_p(out.data_ptr() + 2048), 4096,
                                      vp(status), vp(ws), None)
         assert rc == hs.HS_ERR_ARGUMENT, (firsts, counts)
+
+
+@pytest.mark.parametrize("staged", [False, True])
+def test_digest_sees_every_word(hs, staged):
+    """One flipped bit anywhere in a row fails its record: every 16 B word of
+    the row (each is hashed by its own lane), every bit and byte of a word;
+    rows of equal bytes and untouched neighbours pass."""
+    g = rng(8)
+    n = 320
+    rows = g.integers(0, 256, size=(n, 4096), dtype=np.uint8)
+    rows[300:302], rows[302:304] = 0, 255
+    image = pinned_image(hs, 3, 1, n, 0, rows)
+    raw = image.numpy()
+    flips = [(w, 16 * w + w % 16, w % 8) for w in range(256)]  # record, byte of the row, bit
+    flips += [(256 + i, at, i % 8) for i, at in enumerate((0, 1023, 1024, 2047, 2048, 4095))]
+    for r, at, bit in flips:
+        raw[4096 + r * 4128 + 32 + at] ^= 1 << bit
+    positions = list(range(n))
+    if staged:
+        out, st, _ = runs_fetch(hs, image, 0, positions)
+    else:
+        out, st = cold_fetch(hs, image, 0, positions)
+    assert st["code"] == hs.HS_ERR_CORRUPT and st["k"] == len(flips)
+    for r, at, bit in flips:
+        raw[4096 + r * 4128 + 32 + at] ^= 1 << bit
+    out, st = cold_fetch(hs, image, 0, positions)
+    assert st["code"] == 0 and np.array_equal(out, rows)
