@@ -40,8 +40,9 @@
 //  4. rank:   (rank order only) each id lands at (#head keys above its key)
 //             + (#equal keys in earlier slices) + (its rank among equal keys
 //             of its slice), from histograms over the selected key range.
-// For n <= 32768 steps 2-4 are one launch of a 1024-thread workgroup per
-// head (section 2' below).  Its rank order is a counting sort over the 8192
+// For n <= 65536 steps 2-4 are one launch of a 1024-thread workgroup per
+// head (section 2' below; in rank order up to k = 8192, and up to 13312 past
+// 32768 ids).  Its rank order is a counting sort over the 8192
 // keys from K*'s 256-key bucket upward: the selected (key, id) composites
 // compacted in id order, scattered one per lane into their key's group, and
 // each placed by its rank among its group's ids; a radix sort takes over
@@ -70,12 +71,15 @@ constexpr uint32_t kMaxN = 131072;              // policy/gqa_policy_tests.cpp l
 constexpr uint32_t kMaxHeads = 128;
 constexpr uint32_t kMaxSlices = kMaxN / kSlice;  // 32
 constexpr uint32_t kRankCap = 16384;             // a head's sorted keys staged in LDS
-// per-head path (n <= kHeadMaxN): one 1024-thread workgroup per head
+// per-head path: one 1024-thread workgroup per head, kW membership words of
+// 32 consecutive ids per thread: kW = 1 up to kHeadMaxN ids, 2 up to twice that
 constexpr uint32_t kHThreads = 1024;
 constexpr uint32_t kHWaves = kHThreads / 64;
-constexpr uint32_t kHRun = 32;                     // ids per thread: one membership word
-constexpr uint32_t kHeadMaxN = kHThreads * kHRun;  // 32768
-constexpr uint32_t kHeadMaxK = 8192;               // rank order: selection sorted in LDS
+constexpr uint32_t kHeadMaxN = kHThreads * 32;  // 32768
+constexpr uint32_t kHeadMaxN2 = 2 * kHeadMaxN;  // 65536
+// rank order: the largest selection sorted in LDS (kW = 2: the 20 % cap of
+// 65536 ids is 13107)
+constexpr uint32_t kHeadMaxK = 8192, kHeadMaxK2 = 13312;
 
 // code and k: published by group 0 of the plan launch or head 0 of the
 // per-head launch; head_max: the head-0 maximum order key (the current
@@ -120,7 +124,7 @@ __host__ __device__ SelectPlan plan_select(uint32_t heads, uint32_t n, uint32_t 
     p.off_keys = take(sizeof(uint16_t) * size_t(heads) * p.kcap);
     p.off_m = take(sizeof(uint32_t) * 4 * p.groups);
     p.off_tie = take(sizeof(unsigned long long) * heads);
-    p.key_stride = n <= kHeadMaxN ? (n + 7) / 8 * 8 : 0u;
+    p.key_stride = n <= kHeadMaxN2 ? (n + 7) / 8 * 8 : 0u;
     p.off_key16 = take(sizeof(uint16_t) * size_t(heads) * p.key_stride);
     p.total = at;
     return p;
@@ -1287,36 +1291,56 @@ __global__ void __launch_bounds__(kThreads) slice_select_kernel(SelectArgs a) {
     }
 }
 
-// ---- 2'. per-head select (n <= kHeadMaxN) --------------------------------------
-// One 1024-thread workgroup per head, 32 consecutive ids per thread (one
-// membership word), after the count launch, which also left every score's
+// ---- 2'. per-head select (n <= kHeadMaxN2) -------------------------------------
+// One 1024-thread workgroup per head, kW x 32 consecutive ids per thread (kW
+// membership words), after the count launch, which also left every score's
 // order key in the workspace: k from every head's count, the k-th key from
 // the head's high-byte histograms and a low-byte histogram of its bucket, the
 // ties taken (lowest ids first), then membership and the ids in id order, or,
-// for rank order, the selection (k <= kHeadMaxK) stable-sorted by key in LDS.
+// for rank order, the selection stable-sorted by key in LDS.
 // Every head-wide step is a workgroup step, so plan, select and rank need no
-// launch boundaries between them.
-static_assert(kHeadMaxN / 64 <= kHThreads, "one head-0 tile maximum per thread");
-static_assert(kMaxHeads * (kHeadMaxN / kSlice) <= kHThreads, "one slice count per thread");
+// launch boundaries between them.  Past 32768 ids (kW = 2) the slice
+// launches it replaces were latency chains of their own (plan, select and in
+// rank order rank): score, rank-order cover and union of 48001 tokens take
+// 60.5 us against 83.8, of 65536 60.8 against 77.4, of 33001 49.0 against
+// 69.6; a whole layer (id order) of 65536 tokens 66.0 against 67.4, of 40001
+// 62.8 against 65.1.
+static_assert(kMaxHeads * (kHeadMaxN / kSlice) <= kHThreads, "kW slice counts per thread");
 static_assert(kSortRange % kHThreads == 0, "whole key bins per thread");
 
+// Capacities of one per-head workgroup.  kMaxK: composites in rank order;
+// kRound: composites compacted at a time (kW = 2 compacts each of a thread's
+// words in turn, since the LDS does not hold two lists of kHeadMaxK2); kStage:
+// ids staged in id order.
+template <uint32_t kW>
+struct HeadCaps {
+    static constexpr uint32_t kMaxK = kW == 1 ? kHeadMaxK : kHeadMaxK2;
+    static constexpr uint32_t kRound = kHeadMaxK;
+    static constexpr uint32_t kStage = kW == 1 ? kHeadMaxK : 2 * kHeadMaxK;
+};
+
 // LDS of one per-head workgroup.
-template <bool kRankOrder>
+template <bool kRankOrder, uint32_t kW>
 struct HeadSelectLds {
+    using Caps = HeadCaps<kW>;
     uint32_t hist[2][256];
     uint32_t head_count[kMaxHeads], head_bad[kMaxHeads];
     uint32_t tmp[kHWaves];
     uint32_t sh[8];
-    uint32_t sort_lds[kRankOrder ? 2 * kHeadMaxK + 8 : 1];
+    uint32_t sort_lds[kRankOrder ? Caps::kMaxK + 8 + Caps::kRound : 1];
     alignas(16) uint32_t tables[kRankOrder ? 2 * kSortRange : 1];
-    uint32_t whist[kRankOrder ? kHWaves : 1][256];
-    uint32_t stage[kRankOrder ? 1 : kHeadMaxK];  // id order: the ids before their store
+    // kW = 1: the radix sort's histograms, or a spare word per thread; kW = 2:
+    // the spare words (the histograms take the compacted list's place)
+    uint32_t whist[kRankOrder ? (kW == 1 ? kHWaves : kHThreads / 256) : 1][256];
+    uint32_t stage[kRankOrder ? 1 : Caps::kStage];  // id order: the ids before their store
 };
+static_assert(sizeof(HeadSelectLds<true, 2>) <= 160 * 1024, "one workgroup's LDS");
 
 // The selection of head h of job `job` by one kHThreads workgroup.
-template <bool kRankOrder>
+template <bool kRankOrder, uint32_t kW>
 __device__ __forceinline__ void head_select(const SelectJobs& js, uint32_t h, uint32_t job,
-                                            HeadSelectLds<kRankOrder>& lds) {
+                                            HeadSelectLds<kRankOrder, kW>& lds) {
+    using Caps = HeadCaps<kW>;
     auto& hist = lds.hist;
     auto& head_count = lds.head_count;
     auto& head_bad = lds.head_bad;
@@ -1325,18 +1349,22 @@ __device__ __forceinline__ void head_select(const SelectJobs& js, uint32_t h, ui
     auto& sort_lds = lds.sort_lds;
     auto& tables = lds.tables;
     auto& whist = lds.whist;
-    enum { kCode, kK, kBucket, kAbove, kBucket2, kAbove2, kFlag };
+    enum { kCode, kK, kBucket, kAbove, kBucket2, kAbove2, kFlag, kRounds };
     const SelectArgs a = job_args(js, job);
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t S = a.S, n = a.n, groups = a.heads * S;
-    const uint32_t begin = tid * kHRun, words = (n + 31) / 32;
+    const uint32_t begin = tid * 32 * kW, words = (n + 31) / 32;
 
     // every global read is issued up front: head-0 tile maxima, all slice
     // counts and flags, this head's slice histograms and this thread's keys
     const uint32_t best = a.plan->head_max;  // published by the count launch
-    const uint32_t cnt = load_or_zero(a.g_count, tid, groups);
-    const uint32_t bad = load_or_zero(a.g_bad, tid, groups);
-    constexpr uint32_t kBinLoads = (kHeadMaxN / kSlice) * 256 / kHThreads;  // 2
+    uint32_t cnt[kW], bad[kW];
+#pragma unroll
+    for (uint32_t w = 0; w < kW; ++w) {
+        cnt[w] = load_or_zero(a.g_count, tid + w * kHThreads, groups);
+        bad[w] = load_or_zero(a.g_bad, tid + w * kHThreads, groups);
+    }
+    constexpr uint32_t kBinLoads = kW * (kHeadMaxN / kSlice) * 256 / kHThreads;  // 2 kW
     uint32_t hv[kBinLoads];
 #pragma unroll
     for (uint32_t u = 0; u < kBinLoads; ++u) {
@@ -1344,16 +1372,18 @@ __device__ __forceinline__ void head_select(const SelectJobs& js, uint32_t h, ui
         hv[u] = load_or_zero(a.g_hi + static_cast<size_t>(h * S) * 256, i, S * 256);
     }
     // (key_stride: n rounded up to 8, so at least 8)
-    uint32_t keys[kHRun / 2];
+    uint32_t keys[kW][16];
     const uint16_t* krow = a.g_key16 + static_cast<size_t>(h) * a.key_stride;
 #pragma unroll
-    for (uint32_t v = 0; v < kHRun / 8; ++v) {
-        const uint32_t at = begin + 8 * v;
-        const bool in = at < a.key_stride;
-        const uint4 x = *reinterpret_cast<const uint4*>(krow + (in ? at : a.key_stride - 8));
-        keys[4 * v] = in ? x.x : 0u; keys[4 * v + 1] = in ? x.y : 0u;
-        keys[4 * v + 2] = in ? x.z : 0u; keys[4 * v + 3] = in ? x.w : 0u;
-    }
+    for (uint32_t w = 0; w < kW; ++w)
+#pragma unroll
+        for (uint32_t v = 0; v < 4; ++v) {
+            const uint32_t at = begin + 32 * w + 8 * v;
+            const bool in = at < a.key_stride;
+            const uint4 x = *reinterpret_cast<const uint4*>(krow + (in ? at : a.key_stride - 8));
+            keys[w][4 * v] = in ? x.x : 0u; keys[w][4 * v + 1] = in ? x.y : 0u;
+            keys[w][4 * v + 2] = in ? x.z : 0u; keys[w][4 * v + 3] = in ? x.w : 0u;
+        }
 
     if (tid < 256) hist[0][tid] = hist[1][tid] = 0;
     if (tid < a.heads) head_count[tid] = head_bad[tid] = 0;
@@ -1362,9 +1392,13 @@ __device__ __forceinline__ void head_select(const SelectJobs& js, uint32_t h, ui
         if (tid == 0) sh[kFlag] = 0;
     }
     __syncthreads();
-    if (tid < groups) {
-        atomicAdd(&head_count[tid / S], cnt);
-        atomicOr(&head_bad[tid / S], bad);
+#pragma unroll
+    for (uint32_t w = 0; w < kW; ++w) {
+        const uint32_t i = tid + w * kHThreads;
+        if (i < groups) {
+            atomicAdd(&head_count[i / S], cnt[w]);
+            atomicOr(&head_bad[i / S], bad[w]);
+        }
     }
 #pragma unroll
     for (uint32_t u = 0; u < kBinLoads; ++u)
@@ -1392,7 +1426,10 @@ __device__ __forceinline__ void head_select(const SelectJobs& js, uint32_t h, ui
     const int code = static_cast<int>(sh[kCode]);
     const uint32_t k = sh[kK];
     if (code != HS_OK || k == 0) {  // no stale bitmaps after a failed selection
-        if (a.member && tid < words) a.member[static_cast<size_t>(h) * words + tid] = 0u;
+#pragma unroll
+        for (uint32_t w = 0; w < kW; ++w)
+            if (a.member && kW * tid + w < words)
+                a.member[static_cast<size_t>(h) * words + kW * tid + w] = 0u;
         return;
     }
 
@@ -1405,39 +1442,42 @@ __device__ __forceinline__ void head_select(const SelectJobs& js, uint32_t h, ui
     constexpr uint32_t kSpan = kRankOrder ? kSortRange : 256u;
     uint32_t* table = kRankOrder ? tables : hist[1];
     uint32_t top = 0;  // the largest key counted from the base (rank order)
-    if (kRankOrder && begin + kHRun <= n) {
-        // no branch per key (three VALU instructions and an LDS add, where a
-        // branch costs six and two exec-mask changes): a key outside the
-        // table counts into this lane's own word past it, a cursor word
-        // that the placement writes before it reads any; the largest key
-        // comes from packed 16-bit maxima of the key words
-        const uint32_t lim = kSpan + lane;
-        typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
-        u16x2 pm = __builtin_bit_cast(u16x2, keys[0]);
 #pragma unroll
-        for (uint32_t j = 0; j < kHRun; ++j) {
-            const uint32_t d = half_at(keys, j) - base;  // wraps below the bucket
-            atomicAdd(&table[min(d, lim)], 1u);
-            if (j % 2 == 1 && j > 1)
-                pm = __builtin_elementwise_max(pm, __builtin_bit_cast(u16x2, keys[j / 2]));
-        }
-        top = max(static_cast<uint32_t>(pm.x), static_cast<uint32_t>(pm.y));
-    } else if (begin + kHRun <= n) {  // every thread but a row's last, partial one
+    for (uint32_t w = 0; w < kW; ++w) {
+        const uint32_t at = begin + 32 * w;
+        if (kRankOrder && at + 32 <= n) {
+            // no branch per key (three VALU instructions and an LDS add, where
+            // a branch costs six and two exec-mask changes): a key outside the
+            // table counts into this lane's own word past it, a cursor word
+            // that the placement writes before it reads any; the largest key
+            // comes from packed 16-bit maxima of the key words
+            const uint32_t lim = kSpan + lane;
+            typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+            u16x2 pm = __builtin_bit_cast(u16x2, keys[w][0]);
 #pragma unroll
-        for (uint32_t j = 0; j < kHRun; ++j) {
-            const uint32_t key = half_at(keys, j);
-            const uint32_t d = key - base;  // wraps below the bucket
-            if (d < kSpan) atomicAdd(&table[d], 1u);
-            if (kRankOrder) top = max(top, key);
-        }
-    } else {
+            for (uint32_t j = 0; j < 32; ++j) {
+                const uint32_t d = half_at(keys[w], j) - base;  // wraps below the bucket
+                atomicAdd(&table[min(d, lim)], 1u);
+                if (j % 2 == 1 && j > 1)
+                    pm = __builtin_elementwise_max(pm, __builtin_bit_cast(u16x2, keys[w][j / 2]));
+            }
+            top = max(top, max(static_cast<uint32_t>(pm.x), static_cast<uint32_t>(pm.y)));
+        } else if (at + 32 <= n) {  // every word but a row's last, partial one
 #pragma unroll
-        for (uint32_t j = 0; j < kHRun; ++j) {
-            const uint32_t key = half_at(keys, j);
-            const uint32_t d = key - base;
-            const bool in = begin + j < n;
-            if (in && d < kSpan) atomicAdd(&table[d], 1u);
-            if (kRankOrder && in) top = max(top, key);
+            for (uint32_t j = 0; j < 32; ++j) {
+                const uint32_t key = half_at(keys[w], j);
+                const uint32_t d = key - base;  // wraps below the bucket
+                if (d < kSpan) atomicAdd(&table[d], 1u);
+            }
+        } else {
+#pragma unroll
+            for (uint32_t j = 0; j < 32; ++j) {
+                const uint32_t key = half_at(keys[w], j);
+                const uint32_t d = key - base;
+                const bool in = at + j < n;
+                if (in && d < kSpan) atomicAdd(&table[d], 1u);
+                if (kRankOrder && in) top = max(top, key);
+            }
         }
     }
     if (kRankOrder && top >= base + kSpan) sh[kFlag] = 1u;
@@ -1455,18 +1495,24 @@ __device__ __forceinline__ void head_select(const SelectJobs& js, uint32_t h, ui
     if (tid == 0 && cut_tie && kstar != 0x8000u) atomicAdd(&a.status->boundary_tied_heads, 1u);
     const bool zero_cut = cut_tie && kstar == 0x8000u;
 
-    // this thread's keys above K* and ties, as bit masks over its 32 ids
-    // (bit j = id begin + j, shifted in from the top id down)
-    const uint32_t valid = begin + kHRun <= n ? 0xffffffffu
-                                               : (begin < n ? (1u << (n - begin)) - 1u : 0u);
-    uint32_t above_mask, tie_mask;
-    key_masks(keys, kstar, above_mask, tie_mask);
-    above_mask &= valid;
-    tie_mask &= valid;
-    // one scan of both counts (each total <= 32768 fits its 16 bits): the ties
-    // taken before this thread are min(ties before it, t_need)
-    const uint32_t my_ties = static_cast<uint32_t>(__popc(tie_mask));
-    const uint32_t my_counts = (static_cast<uint32_t>(__popc(above_mask)) << 16) | my_ties;
+    // this thread's keys above K* and ties, as bit masks over each word's 32
+    // ids (bit j = the word's id j, shifted in from the top id down)
+    uint32_t above_mask[kW], tie_mask[kW];
+    uint32_t my_ties = 0, my_above = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kW; ++w) {
+        const uint32_t at = begin + 32 * w;
+        const uint32_t valid = at + 32 <= n ? 0xffffffffu : (at < n ? (1u << (n - at)) - 1u : 0u);
+        key_masks(keys[w], kstar, above_mask[w], tie_mask[w]);
+        above_mask[w] &= valid;
+        tie_mask[w] &= valid;
+        my_ties += static_cast<uint32_t>(__popc(tie_mask[w]));
+        my_above += static_cast<uint32_t>(__popc(above_mask[w]));
+    }
+    // one scan of both counts (an exclusive prefix of either is below 65536,
+    // so it fits its 16 bits): the ties taken before this thread are min(ties
+    // before it, t_need)
+    const uint32_t my_counts = (my_above << 16) | my_ties;
     // Rank order: the counting sort's bins (below) are scanned in the same
     // exchange.  Bins above K*'s hold every key, K*'s bin the t_need ties
     // taken, lower bins nothing.  Thread t owns kPer consecutive bins, thread
@@ -1501,48 +1547,78 @@ __device__ __forceinline__ void head_select(const SelectJobs& js, uint32_t h, ui
     const uint32_t tie_start = both & 0xffffu;
     const uint32_t my_taken = std::min(my_ties, sat_sub(t_need, tie_start));
     uint32_t pos = (both >> 16) + std::min(tie_start, t_need);
-    uint32_t bits32 = above_mask, rest = tie_mask;
-    for (uint32_t t = 0; t < my_taken; ++t) {  // the lowest-id ties first
-        const uint32_t low = rest & (0u - rest);
-        bits32 |= low;
-        rest ^= low;
+    uint32_t bits32[kW], tie_left = my_taken;
+#pragma unroll
+    for (uint32_t w = 0; w < kW; ++w) {
+        bits32[w] = above_mask[w];
+        uint32_t rest = tie_mask[w];
+        const uint32_t take = kW == 1 ? tie_left : std::min(tie_left, static_cast<uint32_t>(__popc(rest)));
+        tie_left -= take;
+        for (uint32_t t = 0; t < take; ++t) {  // the lowest-id ties first
+            const uint32_t low = rest & (0u - rest);
+            bits32[w] |= low;
+            rest ^= low;
+        }
     }
     if (zero_cut) {
         // the ties ranked t_need-1 and t_need: compare their raw bits
         const uint16_t* row = a.scores + static_cast<size_t>(h) * a.stride;
-        uint32_t m = tie_mask;
-        for (uint32_t r = tie_start; m != 0; ++r) {
-            const uint32_t j = static_cast<uint32_t>(__ffs(m)) - 1;
-            m &= m - 1;
-            if (r + 1 == t_need || r == t_need) {
-                uint32_t bits = row[begin + j];
-                if (a.flags & HS_SELECT_SCALE_RAW) bits = scale_raw(bits);
-                note_zero_tie(a, h, bits, r == t_need);
+        uint32_t r = tie_start;
+#pragma unroll
+        for (uint32_t w = 0; w < kW; ++w)
+            for (uint32_t m = tie_mask[w]; m != 0; ++r) {
+                const uint32_t j = static_cast<uint32_t>(__ffs(m)) - 1;
+                m &= m - 1;
+                if (r + 1 == t_need || r == t_need) {
+                    uint32_t bits = row[begin + 32 * w + j];
+                    if (a.flags & HS_SELECT_SCALE_RAW) bits = scale_raw(bits);
+                    note_zero_tie(a, h, bits, r == t_need);
+                }
             }
-        }
     }
-    if (a.member && tid < words) a.member[static_cast<size_t>(h) * words + tid] = bits32;
+#pragma unroll
+    for (uint32_t w = 0; w < kW; ++w)
+        if (a.member && kW * tid + w < words)
+            a.member[static_cast<size_t>(h) * words + kW * tid + w] = bits32[w];
     uint32_t* out = a.ids + static_cast<size_t>(h) * a.ids_stride;
     if constexpr (!kRankOrder) {
-        if (k <= kHeadMaxK) {
+        if (k <= Caps::kStage) {
             // into LDS at their places, then out in row order: the stores of a
             // wave cover 256 consecutive bytes instead of 64 scattered places
             uint32_t* stage = lds.stage;
-            for (uint32_t sel = bits32; sel != 0; sel &= sel - 1)
-                stage[pos++] = begin + static_cast<uint32_t>(__ffs(sel)) - 1;
+#pragma unroll
+            for (uint32_t w = 0; w < kW; ++w)
+                for (uint32_t sel = bits32[w]; sel != 0; sel &= sel - 1)
+                    stage[pos++] = begin + 32 * w + static_cast<uint32_t>(__ffs(sel)) - 1;
             __syncthreads();
             for (uint32_t r = tid; r < k; r += kHThreads) out[r] = stage[r];
         } else {
-            for (uint32_t sel = bits32; sel != 0; sel &= sel - 1)
-                out[pos++] = begin + static_cast<uint32_t>(__ffs(sel)) - 1;
+#pragma unroll
+            for (uint32_t w = 0; w < kW; ++w)
+                for (uint32_t sel = bits32[w]; sel != 0; sel &= sel - 1)
+                    out[pos++] = begin + 32 * w + static_cast<uint32_t>(__ffs(sel)) - 1;
         }
     } else {
-        // Rank order (k <= kHeadMaxK here): a counting sort by key over the
+        // Rank order (k <= Caps::kMaxK here): a counting sort by key over the
         // table's bins (counted and scanned above), larger keys first.
         const uint32_t m = k;
         uint32_t* cursor = tables + kSortRange;
         uint32_t* B = sort_lds;
-        if (sh[kFlag] == 0) {
+        // kW = 2: where each word's composites go in its round's list, and how
+        // many each round holds (a round past the list: the radix sort)
+        uint32_t place = pos, in_round[kW] = {m};
+        bool fits = true;
+        if constexpr (kW == 2) {
+            const uint32_t both_words = static_cast<uint32_t>(__popc(bits32[0])) |
+                                        (static_cast<uint32_t>(__popc(bits32[kW - 1])) << 16);
+            place = block_exclusive_scan<kHThreads>(both_words, tmp);
+            if (tid == kHThreads - 1) sh[kRounds] = place + both_words;
+            __syncthreads();
+            in_round[0] = sh[kRounds] & 0xffffu;
+            in_round[kW - 1] = sh[kRounds] >> 16;
+            fits = in_round[0] <= Caps::kRound && in_round[kW - 1] <= Caps::kRound;
+        }
+        if (sh[kFlag] == 0 && fits) {
             uint32_t run = higher + sum, at[kPer];
 #pragma unroll
             for (uint32_t i = 0; i < kPer; ++i) {
@@ -1566,38 +1642,40 @@ __device__ __forceinline__ void head_select(const SelectJobs& js, uint32_t h, ui
             // spare + sel * gap, gap the bytes from the spare word to the next
             // place in C: one 24-bit multiply-add per id instead of a compare
             // and a select, and one shift-add to move the place on.
-            uint32_t* C = sort_lds + kHeadMaxK + 8;
+            uint32_t* C = sort_lds + Caps::kMaxK + 8;
             static_assert(sizeof(whist) >= kHThreads * sizeof(uint32_t), "a spare word per thread");
-            static_assert(sizeof(HeadSelectLds<kRankOrder>) < (1u << 23), "gap fits 24 signed bits");
-            {
-                char* const spare = reinterpret_cast<char*>(&whist[0][0] + tid);
-                int gap = static_cast<int>(reinterpret_cast<char*>(C + pos) - spare);  // < 0
+            static_assert(sizeof(HeadSelectLds<kRankOrder, kW>) < (1u << 23), "gap fits 24 signed bits");
 #pragma unroll
-                for (uint32_t j = 0; j < kHRun; ++j) {
-                    const uint32_t sel = (bits32 >> j) & 1u;
+            for (uint32_t w = 0; w < kW; ++w) {
+                char* const spare = reinterpret_cast<char*>(&whist[0][0] + tid);
+                const uint32_t at = kW == 1 ? place : (place >> (16 * w)) & 0xffffu;
+                int gap = static_cast<int>(reinterpret_cast<char*>(C + at) - spare);
+#pragma unroll
+                for (uint32_t j = 0; j < 32; ++j) {
+                    const uint32_t sel = (bits32[w] >> j) & 1u;
                     *reinterpret_cast<uint32_t*>(spare + __mul24(static_cast<int>(sel), gap)) =
-                        ((0xffffu - half_at(keys, j)) << 16) | (begin + j);
+                        ((0xffffu - half_at(keys[w], j)) << 16) | (begin + 32 * w + j);
                     gap += static_cast<int>(sel << 2);
                     // opaque, so the place stays in bytes: folded back into
                     // a count of words it costs a shift per id
                     asm("" : "+v"(gap));
                 }
-            }
-            __syncthreads();
-            constexpr uint32_t kDense = kHeadMaxK / kHThreads;
+                __syncthreads();
+                constexpr uint32_t kDense = Caps::kRound / kHThreads;
 #pragma unroll
-            for (uint32_t u = 0; u < kDense; ++u) {
-                const uint32_t q = tid + u * kHThreads;
-                if (q < m) {
-                    const uint32_t e = C[q];
-                    B[atomicAdd(&cursor[0xffffu - (e >> 16) - base], 1u)] = e;
+                for (uint32_t u = 0; u < kDense; ++u) {
+                    const uint32_t q = tid + u * kHThreads;
+                    if (q < in_round[w]) {
+                        const uint32_t e = C[q];
+                        B[atomicAdd(&cursor[0xffffu - (e >> 16) - base], 1u)] = e;
+                    }
                 }
+                __syncthreads();
             }
-            __syncthreads();
             // a composite's place in its group is the number of its group's
             // composites below it; the reads run on past the group, where
             // every composite (later groups: smaller keys; the padding) is larger
-            constexpr uint32_t kPerThread = kHeadMaxK / kHThreads;
+            constexpr uint32_t kPerThread = Caps::kMaxK / kHThreads;
 #pragma unroll
             for (uint32_t u = 0; u < kPerThread; ++u) {
                 const uint32_t q = tid + u * kHThreads;
@@ -1621,23 +1699,31 @@ __device__ __forceinline__ void head_select(const SelectJobs& js, uint32_t h, ui
             // radix sort of the composites written in id order
             uint32_t* A = sort_lds;
 #pragma unroll
-            for (uint32_t j = 0; j < kHRun; ++j) {
-                if ((bits32 >> j) & 1u) {
-                    const uint32_t key = half_at(keys, j);
-                    A[pos++] = ((0xffffu - key) << 16) | (begin + j);
+            for (uint32_t w = 0; w < kW; ++w)
+#pragma unroll
+                for (uint32_t j = 0; j < 32; ++j) {
+                    if ((bits32[w] >> j) & 1u) {
+                        const uint32_t key = half_at(keys[w], j);
+                        A[pos++] = ((0xffffu - key) << 16) | (begin + 32 * w + j);
+                    }
                 }
-            }
             __syncthreads();
-            sort_composites<kHThreads>(A, A + kHeadMaxK, m, whist, tmp);
+            if constexpr (kW == 1) {
+                sort_composites<kHThreads>(A, A + kHeadMaxK, m, whist, tmp);
+            } else {  // the tables and the compacted list are free here
+                static_assert(2 * kSortRange >= Caps::kMaxK && Caps::kRound >= kHWaves * 256, "room for the sort");
+                sort_composites<kHThreads>(A, tables, m,
+                                           reinterpret_cast<uint32_t(*)[256]>(sort_lds + Caps::kMaxK + 8), tmp);
+            }
             for (uint32_t r = tid; r < m; r += kHThreads) out[r] = A[r] & 0xffffu;
         }
     }
 }
 
-template <bool kRankOrder>
+template <bool kRankOrder, uint32_t kW>
 __global__ void __launch_bounds__(kHThreads) head_select_kernel(const SelectJobs js) {
-    __shared__ HeadSelectLds<kRankOrder> lds;
-    head_select<kRankOrder>(js, blockIdx.x, js.order[blockIdx.y], lds);
+    __shared__ HeadSelectLds<kRankOrder, kW> lds;
+    head_select<kRankOrder, kW>(js, blockIdx.x, js.order[blockIdx.y], lds);
 }
 
 // One layer's per-head selection and the next layer's scoring in one launch
@@ -1652,13 +1738,13 @@ template <bool kRankOrder, bool kBatch>
 __global__ void __launch_bounds__(kHThreads)
 select_score_kernel(const SelectJobs js, const ScoreJobs sj) {
     __shared__ union {
-        HeadSelectLds<kRankOrder> select;
+        HeadSelectLds<kRankOrder, 1> select;
         uint4 score[kHWaves][kHalfTileChunks];
     } lds;
     const uint32_t selectors = js.heads * js.count;
     if (blockIdx.x < selectors) {
-        head_select<kRankOrder>(js, blockIdx.x % js.heads, js.order[blockIdx.x / js.heads],
-                                lds.select);
+        head_select<kRankOrder, 1>(js, blockIdx.x % js.heads, js.order[blockIdx.x / js.heads],
+                                   lds.select);
         return;
     }
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1923,22 +2009,28 @@ int check_job(const uint16_t* scores, size_t stride, uint32_t n, const uint32_t*
     return HS_OK;
 }
 
-// The per-head path covers the job: n <= 32768 and, in rank order, a cap
-// whose selection fits the LDS sort.
-bool per_head_path(uint32_t n, float ratio, uint32_t flags) {
-    return n <= kHeadMaxN &&
-           ((flags & HS_SELECT_ID_ORDER) || kmax_of(n, ratio, flags) <= kHeadMaxK);
+// Membership words per thread with which the per-head path covers the job (0:
+// it does not): n ids, and in rank order a cap whose selection fits the LDS
+// sort.
+uint32_t per_head_words(uint32_t n, float ratio, uint32_t flags) {
+    if (n > kHeadMaxN2) return 0;
+    const uint32_t kw = n <= kHeadMaxN ? 1 : 2;
+    const uint32_t max_k = kw == 1 ? kHeadMaxK : kHeadMaxK2;
+    return ((flags & HS_SELECT_ID_ORDER) || kmax_of(n, ratio, flags) <= max_k) ? kw : 0;
 }
 
 // What the launches of a batch need to know about its jobs.
 struct BatchShape {
     uint32_t heads = 0, max_partials = 0, max_groups = 0, max_slices = 0, slices = 0;
     bool any_own_partial = false, all_per_head = true, any_current = false, all_aligned = true;
+    uint32_t head_words = 1;  // per-head path: membership words per thread, 1 or 2
+    // every job on the per-head path with one word per thread (n <= 32768)
+    bool one_word() const { return all_per_head && head_words == 1; }
     // slices per count group: kWideCount when a per-head batch of 16-byte
     // aligned score rows has more (head, slice) pairs than one round of count
     // groups holds (four workgroups on each of 256 CUs)
     uint32_t count_width() const {
-        return all_per_head && all_aligned && slices > 1024 ? kWideCount : 1u;
+        return one_word() && all_aligned && slices > 1024 ? kWideCount : 1u;
     }
     uint32_t count_groups() const {
         const uint32_t r = count_width();
@@ -1956,7 +2048,9 @@ BatchShape batch_shape(const SelectJobs& js) {
         b.slices += p.groups;
         b.any_own_partial |= js.job[j].partial == nullptr;
         b.any_current |= js.job[j].cur_key != nullptr;
-        b.all_per_head &= per_head_path(js.job[j].n, js.ratio, js.flags);
+        const uint32_t kw = per_head_words(js.job[j].n, js.ratio, js.flags);
+        b.all_per_head &= kw != 0;
+        b.head_words = std::max(b.head_words, kw);
         b.all_aligned &= (reinterpret_cast<uintptr_t>(js.job[j].scores) & 15u) == 0 &&
                          js.job[j].stride % 8 == 0 && js.job[j].n >= 8;
     }
@@ -2004,12 +2098,10 @@ int launch_jobs(const SelectJobs& js, hipStream_t stream) {
     const bool id_order = (js.flags & HS_SELECT_ID_ORDER) != 0;
     if (b.all_per_head) {
         // one workgroup per (head, job) finishes the selection
-        if (id_order)
-            hipLaunchKernelGGL(head_select_kernel<false>, dim3(js.heads, js.count), dim3(kHThreads),
-                               0, stream, js);
-        else
-            hipLaunchKernelGGL(head_select_kernel<true>, dim3(js.heads, js.count), dim3(kHThreads),
-                               0, stream, js);
+        const auto kernel = b.head_words == 1
+                                ? (id_order ? head_select_kernel<false, 1> : head_select_kernel<true, 1>)
+                                : (id_order ? head_select_kernel<false, 2> : head_select_kernel<true, 2>);
+        hipLaunchKernelGGL(kernel, dim3(js.heads, js.count), dim3(kHThreads), 0, stream, js);
     } else {
         // one large job: the slice launch chain
         const SelectArgs args = job_args(js, 0);
@@ -2182,7 +2274,7 @@ int launch_select_then_score(const hs_select_job_t* select_jobs, uint32_t select
     rc = check_disjoint(select_jobs, select_count, heads, ratio, flags, score_jobs, score_count);
     if (rc != HS_OK) return rc;
     const BatchShape b = batch_shape(js);
-    if (!b.all_per_head) {  // the slice chain: the two calls in turn
+    if (!b.one_word()) {  // no shared launch: the two calls in turn
         rc = launch_jobs(js, stream);
         return rc != HS_OK ? rc : launch_score_batched(score_jobs, score_count, stream);
     }

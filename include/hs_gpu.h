@@ -148,8 +148,9 @@ int hs_gqa_score_batched(const hs_score_job_t *jobs, uint32_t count, void *strea
  * initialisation needed).
  * head0_partial_dev: NULL, or the per-tile maxima from hs_gqa_score over
  * the same raw scores (skips one pass over head 0).
- * One call is 2 launches on `stream` when n <= 32768 (and, in rank
- * order, floor(n*ratio) <= 8192), otherwise 3 (4 in rank order); +1
+ * One call is 2 launches on `stream` when n <= 65536 (and, in rank
+ * order, floor(n*ratio) <= 8192, or 13312 past n = 32768), otherwise 3 (4
+ * in rank order); +1
  * without head0_partial_dev.  Calls sharing a workspace must be ordered on
  * one stream.
  * HS_SELECT_COUNTED: the first (count) launch of this selection already ran
@@ -173,8 +174,8 @@ int hs_gqa_select(const uint16_t *scores_dev, uint32_t heads, size_t stride,
 /* Batched selection: up to 16 independent selections (the decode sequences
  * of a batch: each its own scores, n, outputs and workspace of
  * hs_gqa_select_workspace_bytes(heads, n)) sharing heads, alpha, ratio and
- * flags, each with hs_gqa_select's semantics.  When every job has n <= 32768
- * (and, in rank order, floor(n*ratio) <= 8192) one launch per phase serves
+ * flags, each with hs_gqa_select's semantics.  When every job takes the
+ * 2-launch form of hs_gqa_select one launch per phase serves
  * the whole batch; otherwise the jobs run one after another. */
 typedef struct {
     const uint16_t *scores;          /* F16 [heads][stride]                  */

@@ -390,3 +390,59 @@ def test_random_batch_sweep_against_oracle(hs, port):
             assert st["k"] == k and st["boundary_tied_heads"] == tied
             assert np.array_equal(from_dev(counts), pcounts)
             assert np.array_equal(from_dev(ids)[:, :k], pids)
+
+
+@pytest.mark.parametrize("n", [32769, 40001, 65535, 65536])
+@pytest.mark.parametrize("kind", ["gaussian", "ties", "equal", "wide", "first_words", "zeros"])
+def test_two_words_per_thread(hs, port, n, kind):
+    # the per-head launch past 32768 ids: two membership words per thread, the
+    # rank-order composites compacted a word at a time (first_words: more
+    # than a round's list holds, so the radix sort takes over, as it does for
+    # long runs of equal keys and wide key ranges), ties and a signed zero at
+    # the cut, all ids equal, and members
+    g = rng(n + len(kind))
+    heads, alpha, ratio = 4, 5.0, 0.2
+    s = f16_bits(g.standard_normal((heads, n)) * 2.0)
+    if kind == "ties":
+        s, alpha = f16_bits(g.integers(-400, 400, size=(heads, n)) / 32.0), 20.0
+    elif kind == "equal":
+        s[:], alpha = hb(0.5), 0.0
+    elif kind == "wide":
+        s = g.integers(0x0400, 0x7BFF, size=(heads, n)).astype(np.uint16)
+        alpha = 70000.0
+    elif kind == "first_words":  # the largest scores in every thread's first word
+        big = f16_bits(30.0 + np.abs(g.standard_normal((heads, n))))
+        s = np.where((np.arange(n) & 63) < 32, big, s)
+        alpha = 100.0
+    elif kind == "zeros":
+        s = np.where(g.random((heads, n)) < 0.5, 0x8000, 0).astype(np.uint16)
+        s[:, ::11] = hb(3.0)
+        alpha = 5.0
+    # (a count past 65504 rounds beyond F16: those cases count in FP32)
+    rc, k, ids, _, _ = port.select(s, heads, n, n, alpha, ratio, True)
+    assert rc == 0 and 0 < k <= 13107
+    check_against_port(hs, port, s, heads, n, n, alpha, ratio, True)
+    member = torch.zeros(heads * ((n + 31) // 32), dtype=torch.int32, device="cuda")
+    gpu_select(hs, s, heads, n, n, alpha, ratio, fp32_counts=True, member=member)
+    assert np.array_equal(from_dev(member).view(np.uint32).reshape(heads, -1), member_from_ids(ids, n))
+
+
+def test_mixed_word_counts_in_a_batch(hs, port):
+    # one launch for jobs on both sides of 32768 ids; a cap too large for the
+    # rank-order sort sends the jobs to their own launches
+    g = rng(515)
+    for ratio in (0.2, 0.3):
+        raws, jobs = [], []
+        for n in (1000, 32768, 32776, 50000, 65536):
+            raw = f16_bits(g.standard_normal((32, n)) * 20.0)
+            raws.append(raw)
+            jobs.append(dict(scores=to_dev(raw.reshape(-1)).view(32, n), n=n))
+        for id_order in (False, True):
+            res = hs.ops.select_batched(jobs, 32, 4.0, ratio, scale_raw=True, id_order=id_order)
+            for raw, (ids, counts, _, status) in zip(raws, res):
+                n = raw.shape[1]
+                rc, k, pids, pcounts, tied = port.select(port.scale(raw), 32, n, n, 4.0, ratio)
+                st = hs.ops.read_status(status)
+                assert rc == 0 and st["code"] == 0 and st["k"] == k and st["boundary_tied_heads"] == tied
+                assert np.array_equal(from_dev(counts), pcounts)
+                assert np.array_equal(from_dev(ids)[:, :k], np.sort(pids, axis=1) if id_order else pids)
