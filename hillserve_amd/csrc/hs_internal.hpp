@@ -40,12 +40,23 @@ inline hipStream_t as_stream(void* stream) { return static_cast<hipStream_t>(str
 // Round a byte count up to 256 B so workspace slices stay aligned.
 inline size_t align256(size_t bytes) { return (bytes + 255) & ~size_t(255); }
 
+// Words that hs_decode_layer's scoring launch clears for the selection that
+// follows it: 32 published counts, 32 tie records of 8 bytes and the status's
+// tied-head count (all null: nothing to clear).
+struct SelectExchange {
+    uint32_t* published = nullptr;
+    uint32_t* ties = nullptr;
+    uint32_t* tied_heads = nullptr;
+};
+
 // ---- launch wrappers implemented in the .hip translation units ----------
-// With qf and logits (both or neither): the attention logits in the same pass.
+// With qf and logits (both or neither): the attention logits in the same pass,
+// and `clear` cleared.
 int launch_score(const uint16_t* q, const uint16_t* keys, size_t stride_words,
                  const int32_t* rows, uint32_t pool_rows, uint32_t tokens, uint16_t* scores,
                  size_t score_stride, uint32_t* head0_partial, hipStream_t stream,
-                 const float* qf = nullptr, float* logits = nullptr, size_t logit_stride = 0);
+                 const float* qf = nullptr, float* logits = nullptr, size_t logit_stride = 0,
+                 const SelectExchange& clear = SelectExchange{});
 
 int launch_score_batched(const hs_score_job_t* jobs, uint32_t count, hipStream_t stream);
 
@@ -54,6 +65,16 @@ int launch_select(const uint16_t* scores, uint32_t heads, size_t stride, uint32_
                   float alpha, float ratio, uint32_t flags, const uint32_t* head0_partial,
                   uint32_t* ids, size_t ids_stride, uint32_t* counts, uint32_t* member,
                   hs_status_t* status, void* workspace, hipStream_t stream);
+// The selection of hs_decode_layer (32 heads, stride n, id order) after a scoring
+// launch that cleared select_exchange's words.  wait_ticks (of 10 ns): how long
+// a workgroup of the short-sequence launch waits for the other heads' counts
+// before it counts the missing heads itself.
+constexpr uint32_t kExchangeTicks = 5000;
+int launch_layer_select(const uint16_t* scores, uint32_t n, float alpha, float ratio, uint32_t flags,
+                        const uint32_t* head0_partial, uint32_t* ids, size_t ids_stride,
+                        uint32_t* counts, uint32_t* member, hs_status_t* status, void* workspace,
+                        hipStream_t stream, uint32_t wait_ticks = kExchangeTicks);
+SelectExchange select_exchange(uint32_t n, float ratio, uint32_t flags, hs_status_t* status, void* workspace);
 // launch_select's host checks only (nothing enqueued)
 int check_select(const uint16_t* scores, uint32_t heads, size_t stride, uint32_t n, float alpha,
                  float ratio, uint32_t flags, const uint32_t* head0_partial, uint32_t* ids,

@@ -194,10 +194,11 @@ int decode_layer(const uint16_t* q16_dev, const float* q32_dev, const uint8_t* k
     // (both queries are known when a layer is scored at its own step), so the
     // attention reads only the selected V rows.
     rc = launch_score(q16_dev, reinterpret_cast<const uint16_t*>(k_pool_dev), row_bytes / 2,
-                      row_of_id_dev, pool_rows, n, scores_dev, n, partial, s, q32_dev, logits, n);
+                      row_of_id_dev, pool_rows, n, scores_dev, n, partial, s, q32_dev, logits, n,
+                      select_exchange(n, ratio, sel_flags, status_dev, ws + p.off_select));
     if (rc != HS_OK) return rc;
-    rc = launch_select(scores_dev, 32, n, n, alpha, ratio, sel_flags, partial, ids_dev, ids_stride,
-                       counts_dev, member, status_dev, ws + p.off_select, s);
+    rc = launch_layer_select(scores_dev, n, alpha, ratio, sel_flags, partial, ids_dev, ids_stride,
+                             counts_dev, member, status_dev, ws + p.off_select, s);
     if (rc != HS_OK) return rc;
     return launch_attention_logits(logits, n, v_pool_dev, row_bytes, row_of_id_dev, pool_rows, member,
                                    n, out_dev, ws + p.off_attn, s);

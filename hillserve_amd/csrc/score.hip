@@ -71,7 +71,13 @@ score_kernel(const ScoreJobs jobs, const int32_t* __restrict__ rows, uint32_t po
 template <bool kRows, bool kStream>
 __global__ void __launch_bounds__(kWavesPerBlock * 64) __attribute__((amdgpu_waves_per_eu(4)))
 score_logits_kernel(const ScoreJobs jobs, const int32_t* __restrict__ rows, uint32_t pool_rows,
-                    const LogitsOut lo) {
+                    const LogitsOut lo, const SelectExchange clear) {
+    if (!kStream && clear.published && blockIdx.x == 0) {  // for the selection that follows
+        const uint32_t tid = threadIdx.x;
+        if (tid < 32) clear.published[tid] = 0;
+        if (tid < 64) clear.ties[tid] = 0;
+        if (tid == 0) *clear.tied_heads = 0;
+    }
     __shared__ uint4 lds[kWavesPerBlock][kHalfTileChunks];
     __shared__ uint4 qstage[kWavesPerBlock][8 * 16];
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -92,7 +98,7 @@ uint32_t score_grid(uint32_t ids) {
 int launch_score(const uint16_t* q, const uint16_t* keys, size_t stride_words,
                  const int32_t* rows, uint32_t pool_rows, uint32_t tokens, uint16_t* scores,
                  size_t score_stride, uint32_t* head0_partial, hipStream_t stream,
-                 const float* qf, float* logits, size_t logit_stride) {
+                 const float* qf, float* logits, size_t logit_stride, const SelectExchange& clear) {
     if (!q || !keys || !scores) return reject("score: null pointer");
     if ((qf == nullptr) != (logits == nullptr)) return reject("score: logits need the F32 query");
     if (logits && (logit_stride < tokens || logit_stride > 0xffffffffu))
@@ -123,7 +129,8 @@ int launch_score(const uint16_t* q, const uint16_t* keys, size_t stride_words,
     if (logits) {
         const auto kernel = rows ? (streamed ? score_logits_kernel<true, true> : score_logits_kernel<true, false>)
                                  : (streamed ? score_logits_kernel<false, true> : score_logits_kernel<false, false>);
-        hipLaunchKernelGGL(kernel, grid, block, 0, stream, jobs, rows, rows ? pool_rows : 0u, lo);
+        hipLaunchKernelGGL(kernel, grid, block, 0, stream, jobs, rows, rows ? pool_rows : 0u, lo,
+                           clear);
     } else {
         const auto kernel = rows ? (streamed ? score_kernel<true, false, true> : score_kernel<true, false, false>)
                                  : (streamed ? score_kernel<false, false, true> : score_kernel<false, false, false>);

@@ -357,6 +357,33 @@ __device__ void find_bucket(const uint32_t* hist, uint32_t need, uint32_t* out_b
     }
 }
 
+// find_bucket by every wave for itself, the result in registers (no barrier
+// to publish it).
+__device__ __forceinline__ void find_bucket_wave(const uint32_t* hist, uint32_t need,
+                                                 uint32_t& bucket, uint32_t& above) {
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t local[4], sum = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+        local[j] = hist[255 - (4 * lane + j)];
+        sum += local[j];
+    }
+    const uint32_t x = wave_inclusive_sum_u32(sum);
+    uint32_t running = x - sum, b = 0, at = 0;
+    const bool here = running < need && need <= x;
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {  // the first j at which the count reaches `need`
+        if (running < need) {
+            b = 255 - (4 * lane + j);
+            at = running;
+        }
+        running += local[j];
+    }
+    const int src = __ffsll(static_cast<long long>(__ballot(here))) - 1;
+    bucket = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(b), src));
+    above = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(at), src));
+}
+
 // Lanes of the wave holding the same 8-bit digit (restricted to `valid`).
 __device__ __forceinline__ uint64_t match_digit(uint32_t digit, bool valid) {
     uint64_t m = __ballot(valid);
@@ -638,11 +665,13 @@ struct CountLds {
 // covers whole consecutive lines.  kR > 1 only for batches whose score rows
 // are all 16-byte aligned with n >= 8 (checked by the host).  kCurrent: some
 // job of the batch completes its current token (waves 0 and 1 of a group
-// score its column; batches without one compile that part out).
-template <bool kCurrent, uint32_t kR>
+// score its column; batches without one compile that part out).  kAligned:
+// every job's score rows are 16-byte aligned with n >= 8 (the host's check).
+template <bool kCurrent, uint32_t kR, bool kAligned>
 __device__ __forceinline__ void count_group(const SelectJobs& js, uint32_t g, uint32_t job,
                                             CountLds& lds) {
     static_assert(kR == 1 || kR == 2 || kR == kWideCount, "packed slice counts");
+    static_assert(kR == 1 || kAligned, "wide groups read whole words");
     static_assert(kSlice < 65536, "a slice count fits 16 bits");
     auto& whist = lds.whist;
     auto& tmp = lds.tmp;
@@ -658,7 +687,7 @@ __device__ __forceinline__ void count_group(const SelectJobs& js, uint32_t g, ui
     uint32_t pv[kLoads];
     partial_loads<kLoads>(a, pv);
     uint32_t packed[kR][kRun / 2];  // ids past n (slices past S) read as zeros
-    load_runs<kRun, kR, kSlice, (kR > 1), false>(a, h, first * kSlice + tid * kRun, packed);
+    load_runs<kRun, kR, kSlice, kAligned, false>(a, h, first * kSlice + tid * kRun, packed);
     const bool scale = (a.flags & HS_SELECT_SCALE_RAW) != 0;
     uint32_t best = 0;
 #pragma unroll
@@ -789,10 +818,10 @@ __device__ __forceinline__ void count_group(const SelectJobs& js, uint32_t g, ui
     }
 }
 
-template <bool kCurrent, uint32_t kR>
+template <bool kCurrent, uint32_t kR, bool kAligned>
 __global__ void __launch_bounds__(kThreads) count_kernel(const SelectJobs js) {
     __shared__ CountLds lds;
-    count_group<kCurrent, kR>(js, blockIdx.x, blockIdx.y, lds);
+    count_group<kCurrent, kR, kAligned>(js, blockIdx.x, blockIdx.y, lds);
 }
 
 // k from every head's count and nonfinite flag (policy/gqa_policy.cpp:51-63),
@@ -1726,6 +1755,210 @@ __global__ void __launch_bounds__(kHThreads) head_select_kernel(const SelectJobs
     head_select<kRankOrder, kW>(js, blockIdx.x, js.order[blockIdx.y], lds);
 }
 
+// ---- 2''. short sequences: count and select in one launch ------------------------
+// n <= kSmallMaxN, id order, one job, after a scoring launch of the same call
+// (hs_decode_layer) that cleared the exchange words.  One workgroup per head,
+// kRun consecutive ids per thread: it scales and counts its head, publishes
+// (count, nonfinite flag) in the head's word, gathers the other heads' words
+// while its own histogram is summed, and selects as the per-head launch does,
+// keys still in registers.  A word is complete in one relaxed agent-scope
+// store (no cache write-back); the wait for the others is bounded, and a
+// head still missing then is counted by the workgroup itself, so a workgroup
+// finishes whatever else the device runs.
+// Latency-bound: the count launch it saves is a launch and a memory round
+// trip, while its arithmetic (8 ids per thread) is little: a layer of 1024
+// tokens takes 22.2 us against 27.8, of 4096 23.8 against 28.5, of 8192 28.1
+// against 31.7.  At 16384 ids (512 threads of 32) it gained 0.7 us and at 12288
+// it lost 0.6, so the line is 8192.
+constexpr uint32_t kSmallMaxN = 8192;
+constexpr uint32_t kPublished = 0x80000000u, kPublishedBad = 0x40000000u;
+
+__device__ __forceinline__ uint64_t realtime_ticks() { return __builtin_amdgcn_s_memrealtime(); }
+
+// One head's run of this thread: scaled order keys into keyw, the number of
+// scores >= the threshold, nonfinite scores flagged; with kOwn each key's high
+// byte into the histogram.
+template <bool kOwn>
+__device__ __forceinline__ uint32_t small_count(const SelectArgs& a, const uint32_t (&packed)[kRun / 2],
+                                                uint32_t begin, float thr, uint32_t kthr,
+                                                uint32_t* hist, uint32_t (&keyw)[kRun / 2], bool& bad) {
+    uint32_t special = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kRun / 2; ++w) special |= (packed[w] & 0x7c007c00u) + 0x04000400u;
+    if (kOwn && (special & 0x80008000u) == 0 && begin + kRun <= a.n)  // (as in count_group)
+        return count_clean_run<true>(packed, kthr, hist, keyw);
+    uint32_t count = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < kRun; ++j) {
+        const uint32_t b = scale_raw(half_at(packed, j)), key = order_key(b);
+        keyw[j >> 1] |= key << ((j & 1u) * 16u);
+        if (begin + j < a.n) {
+            if (!finite_half(b)) {
+                bad = true;
+            } else {
+                count += h2f(b) >= thr ? 1u : 0u;
+                if (kOwn) atomicAdd(&hist[key >> 8], 1u);
+            }
+        }
+    }
+    return count;
+}
+
+template <uint32_t kT, bool kAligned>
+__global__ void __launch_bounds__(kT) small_select_kernel(const SelectJobs js, uint32_t wait_ticks) {
+    static_assert(kT * kRun <= kSmallMaxN && kT >= 256, "one run per thread");
+    __shared__ uint32_t whist[kCountHist], hist[2][256];
+    __shared__ uint32_t head_count[kMaxHeads], head_bad[kMaxHeads];
+    __shared__ uint32_t tmp[kT / 64], sh[4];
+    __shared__ uint64_t missing[2];
+    __shared__ uint32_t stage[kT * kRun];
+    enum { kCode, kK, kBucket, kAbove };
+    const SelectArgs a = job_args(js, 0);
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, h = blockIdx.x;
+    const uint32_t n = a.n, begin = tid * kRun, words = (n + 31) / 32;
+    uint32_t* const published = a.g_count;  // [heads], zero before this launch
+    // the tile maxima and this thread's run, requested before any is used
+    // (at most 128 maxima: one per thread)
+    uint32_t best = a.partial[min(tid, a.partials - 1u)];
+    uint32_t packed[kRun / 2];
+    load_runs<kRun, 1, 0, kAligned, false>(a, h, begin, reinterpret_cast<uint32_t (&)[1][kRun / 2]>(packed));
+    for (uint32_t i = tid; i < kCountHist; i += kT) whist[i] = 0;
+    if (tid < 256) hist[1][tid] = 0;
+    best = block_max<kT>(best, tmp);  // its barriers also order the clears
+    const float thr = threshold_from_key(best, true, a.alpha);
+    const uint32_t kthr = threshold_key_from_key(best, true, a.alpha);
+    uint32_t keyw[kRun / 2] = {};
+    bool my_bad = false;
+    const uint32_t mine = small_count<true>(a, packed, begin, thr, kthr,
+                                            whist + (tid & (kCountCopies - 1)) * kCountCopyStride, keyw, my_bad);
+    // (count <= 8192 per head; the flag rides above it)
+    const uint32_t total = block_sum<kT>(mine + (my_bad ? 0x10000u : 0u), tmp);
+    if (wave == 0) {
+        if (lane == 0)
+            __hip_atomic_store(&published[h], kPublished | (total >> 16 ? kPublishedBad : 0u) | (total & 0xffffu),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint64_t start = realtime_ticks();
+        uint32_t word[kMaxHeads / 64];
+        uint64_t left[kMaxHeads / 64];
+        bool wait = true;
+        while (wait) {
+            wait = false;
+#pragma unroll
+            for (uint32_t u = 0; u < kMaxHeads / 64; ++u) {
+                const uint32_t hh = lane + 64 * u;
+                word[u] = hh < a.heads ? __hip_atomic_load(&published[hh], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                                       : kPublished;
+                left[u] = __ballot(!(word[u] & kPublished));
+                wait |= left[u] != 0;
+            }
+            if (realtime_ticks() - start >= wait_ticks) break;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kMaxHeads / 64; ++u) {
+            const uint32_t hh = lane + 64 * u;
+            if (hh < a.heads) {
+                head_count[hh] = word[u] & 0xffffu;
+                head_bad[hh] = (word[u] & kPublishedBad) ? 1u : 0u;
+            }
+            if (lane == 0) missing[u] = left[u];
+        }
+    } else {
+        for (uint32_t i = tid - 64; i < 256; i += kT - 64) {
+            uint32_t c = 0;
+#pragma unroll
+            for (uint32_t k = 0; k < kCountCopies; ++k) c += whist[k * kCountCopyStride + i];
+            hist[0][i] = c;
+        }
+    }
+    __syncthreads();
+    for (uint32_t u = 0; u < kMaxHeads / 64; ++u)
+        for (uint64_t rest = missing[u]; rest != 0; rest &= rest - 1) {  // (uniform; rare)
+            const uint32_t hh = 64 * u + static_cast<uint32_t>(__ffsll(static_cast<long long>(rest))) - 1;
+            uint32_t other[kRun / 2], unused[kRun / 2] = {};
+            load_runs<kRun, 1, 0, kAligned, false>(a, hh, begin, reinterpret_cast<uint32_t (&)[1][kRun / 2]>(other));
+            bool its_bad = false;
+            const uint32_t c = small_count<false>(a, other, begin, thr, kthr, nullptr, unused, its_bad);
+            const uint32_t t = block_sum<kT>(c + (its_bad ? 0x10000u : 0u), tmp);
+            if (tid == 0) {
+                head_count[hh] = t & 0xffffu;
+                head_bad[hh] = t >> 16 ? 1u : 0u;
+            }
+        }
+    __syncthreads();
+    if (wave == 0) {
+        uint32_t k = 0;
+        const int code = derive_k(a, head_count, head_bad, thr, k);
+        if (lane == 0) {
+            sh[kCode] = static_cast<uint32_t>(code);
+            sh[kK] = k;
+            if (h == 0) {
+                a.status->code = code;
+                a.status->k = code == HS_OK ? k : 0u;
+                a.status->head0_max_key = best;
+            }
+        }
+    }
+    if (h == 0 && tid < a.heads && a.counts_out) a.counts_out[tid] = head_count[tid];
+    __syncthreads();
+    const int code = static_cast<int>(sh[kCode]);
+    const uint32_t k = sh[kK];
+    uint32_t* member = a.member + static_cast<size_t>(h) * words;
+    if (code != HS_OK || k == 0) {  // no stale bitmaps after a failed selection
+        if ((tid & 3u) == 0 && begin / 32 < words) member[begin / 32] = 0u;
+        return;
+    }
+    uint32_t hi, above_hi, lo, above_lo;
+    find_bucket_wave(hist[0], k, hi, above_hi);
+#pragma unroll
+    for (uint32_t j = 0; j < kRun; ++j) {
+        const uint32_t key = half_at(keyw, j);
+        if (begin + j < n && (key >> 8) == hi) atomicAdd(&hist[1][key & 255u], 1u);
+    }
+    __syncthreads();
+    find_bucket_wave(hist[1], k - above_hi, lo, above_lo);
+    const uint32_t kstar = (hi << 8) | lo, c_above = above_hi + above_lo, c_equal = hist[1][lo];
+    const uint32_t t_need = k - c_above;  // ties taken, lowest ids first (>= 1)
+    const bool cut_tie = k < n && c_above + c_equal > k;
+    if (tid == 0 && cut_tie && kstar != 0x8000u) atomicAdd(&a.status->boundary_tied_heads, 1u);
+    const bool zero_cut = cut_tie && kstar == 0x8000u;  // (as in head_select)
+    uint32_t bits8 = 0, ties8 = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < kRun; ++j) {
+        const uint32_t key = half_at(keyw, j);
+        const bool in = begin + j < n;
+        bits8 |= (in && key > kstar ? 1u : 0u) << j;
+        ties8 |= (in && key == kstar ? 1u : 0u) << j;
+    }
+    const uint32_t my_ties = static_cast<uint32_t>(__popc(ties8));
+    const uint32_t both = block_exclusive_scan<kT>((static_cast<uint32_t>(__popc(bits8)) << 16) | my_ties, tmp);
+    const uint32_t tie_start = both & 0xffffu;
+    const uint32_t my_taken = std::min(my_ties, sat_sub(t_need, tie_start));
+    uint32_t pos = (both >> 16) + std::min(tie_start, t_need), rest = ties8;
+    for (uint32_t t = 0; t < my_taken; ++t) {  // the lowest-id ties first
+        const uint32_t low = rest & (0u - rest);
+        bits8 |= low;
+        rest ^= low;
+    }
+    if (zero_cut) {
+        uint32_t r = tie_start;
+        for (uint32_t m = ties8; m != 0; m &= m - 1, ++r)
+            if (r + 1 == t_need || r == t_need) {
+                const uint32_t j = static_cast<uint32_t>(__ffs(m)) - 1;
+                const uint32_t bits = scale_raw(a.scores[static_cast<size_t>(h) * a.stride + begin + j]);
+                note_zero_tie(a, h, bits, r == t_need);
+            }
+    }
+    uint32_t word = bits8 << (8u * (tid & 3u));
+    word |= __shfl_xor(word, 1, 64);
+    word |= __shfl_xor(word, 2, 64);
+    if ((tid & 3u) == 0 && begin / 32 < words) member[begin / 32] = word;
+    for (uint32_t sel = bits8; sel != 0; sel &= sel - 1)
+        stage[pos++] = begin + static_cast<uint32_t>(__ffs(sel)) - 1;
+    __syncthreads();
+    uint32_t* out = a.ids + static_cast<size_t>(h) * a.ids_stride;
+    for (uint32_t r = tid; r < k; r += kT) out[r] = stage[r];
+}
+
 // One layer's per-head selection and the next layer's scoring in one launch
 // (the early history preparation of runtime/gqa_executor.cpp:291-295 and
 // policy/full_gqa_runtime.cpp:493-496, where the next layer's history is
@@ -1948,7 +2181,7 @@ __global__ void __launch_bounds__(kThreads) rank_kernel(SelectArgs a) {
 // heads x 4 channel groups) and the next layer's selection count (the
 // others: (head, slice) groups x jobs) in one launch; both are short and
 // latency-bound, and neither reads what the other writes.
-template <bool kCurrent, uint32_t kR>
+template <bool kCurrent, uint32_t kR, bool kAligned>
 __global__ void __launch_bounds__(kThreads)
 combine_count_kernel(const float* __restrict__ part, uint32_t chunks, float* __restrict__ out,
                      const SelectJobs js, uint32_t groups) {
@@ -1963,7 +2196,7 @@ combine_count_kernel(const float* __restrict__ part, uint32_t chunks, float* __r
         return;
     }
     const uint32_t b = blockIdx.x - kMergers;
-    count_group<kCurrent, kR>(js, b % groups, b / groups, lds.count);
+    count_group<kCurrent, kR, kAligned>(js, b % groups, b / groups, lds.count);
 }
 
 }  // namespace
@@ -2057,15 +2290,6 @@ BatchShape batch_shape(const SelectJobs& js) {
     return b;
 }
 
-template <uint32_t kR>
-void launch_count_kernel(const SelectJobs& js, const BatchShape& b, hipStream_t stream) {
-    const dim3 grid(b.count_groups(), js.count);
-    if (b.any_current)
-        hipLaunchKernelGGL((count_kernel<true, kR>), grid, dim3(kThreads), 0, stream, js);
-    else
-        hipLaunchKernelGGL((count_kernel<false, kR>), grid, dim3(kThreads), 0, stream, js);
-}
-
 // The head-0 maxima (jobs without the scorer's) and the count launch, unless
 // hs_gqa_attention_then_count ran them (HS_SELECT_COUNTED).
 void launch_counts(const SelectJobs& js, const BatchShape& b, hipStream_t stream) {
@@ -2073,10 +2297,15 @@ void launch_counts(const SelectJobs& js, const BatchShape& b, hipStream_t stream
     if (b.any_own_partial)
         hipLaunchKernelGGL(head0_max_kernel, dim3((b.max_partials + 3) / 4, js.count), dim3(256), 0,
                            stream, js);
-    if (b.count_width() == kWideCount)
-        launch_count_kernel<kWideCount>(js, b, stream);
-    else
-        launch_count_kernel<1>(js, b, stream);
+    const bool wide = b.count_width() == kWideCount;
+    const auto kernel =
+        b.any_current ? (wide            ? count_kernel<true, kWideCount, true>
+                         : b.all_aligned ? count_kernel<true, 1, true>
+                                         : count_kernel<true, 1, false>)
+                      : (wide            ? count_kernel<false, kWideCount, true>
+                         : b.all_aligned ? count_kernel<false, 1, true>
+                                         : count_kernel<false, 1, false>);
+    hipLaunchKernelGGL(kernel, dim3(b.count_groups(), js.count), dim3(kThreads), 0, stream, js);
 }
 
 // Launches for the checked jobs of `js`.  Batches whose jobs all take the
@@ -2239,6 +2468,52 @@ int launch_select(const uint16_t* scores, uint32_t heads, size_t stride, uint32_
     return launch_jobs(js, stream);
 }
 
+// The selection of hs_decode_layer.  Its scoring launch has cleared
+// select_exchange's words, so up to kSmallMaxN tokens one launch counts and
+// selects.
+int launch_layer_select(const uint16_t* scores, uint32_t n, float alpha, float ratio, uint32_t flags,
+                        const uint32_t* head0_partial, uint32_t* ids, size_t ids_stride,
+                        uint32_t* counts, uint32_t* member, hs_status_t* status, void* workspace,
+                        hipStream_t stream, uint32_t wait_ticks) {
+    if (n > kSmallMaxN)
+        return launch_select(scores, 32, n, n, alpha, ratio, flags, head0_partial, ids, ids_stride,
+                             counts, member, status, workspace, stream);
+    SelectJobs js{};
+    js.count = 1;
+    js.heads = 32;
+    js.flags = flags;
+    js.alpha = alpha;
+    js.ratio = ratio;
+    const int rc = check_job(scores, n, n, head0_partial, ids, ids_stride, counts, member, status,
+                             workspace, ratio, flags, js.job[0]);
+    if (rc != HS_OK) return rc;
+    // the fewest waves that hold the ids: each of the kernel's barriers waits
+    // for all of a workgroup's (n = 4096: 23.8 us a layer with 512 threads,
+    // 25.4 with 1024, 24.2 with 256 of two runs each)
+    const uint32_t threads = n <= 256 * kRun ? 256u : n <= 512 * kRun ? 512u : 1024u;
+    const bool aligned = (reinterpret_cast<uintptr_t>(scores) & 15u) == 0 && n % 8 == 0;
+    const auto kernel =
+        aligned ? (threads == 256   ? small_select_kernel<256, true>
+                   : threads == 512 ? small_select_kernel<512, true>
+                                    : small_select_kernel<1024, true>)
+                : (threads == 256   ? small_select_kernel<256, false>
+                   : threads == 512 ? small_select_kernel<512, false>
+                                    : small_select_kernel<1024, false>);
+    hipLaunchKernelGGL(kernel, dim3(32), dim3(threads), 0, stream, js, wait_ticks);
+    const hipError_t st = hipGetLastError();
+    return st == hipSuccess ? HS_OK : hip_fail(st, "select launch");
+}
+
+// What the scoring launch before launch_layer_select clears: the published
+// counts, the tie records and the tied-head count.
+SelectExchange select_exchange(uint32_t n, float ratio, uint32_t flags, hs_status_t* status, void* workspace) {
+    if (n > kSmallMaxN) return SelectExchange{};
+    const SelectPlan p = plan_select(32, n, kmax_of(n, ratio, flags));
+    char* ws = static_cast<char*>(workspace);
+    return SelectExchange{reinterpret_cast<uint32_t*>(ws + p.off_count), reinterpret_cast<uint32_t*>(ws + p.off_tie),
+                          &status->boundary_tied_heads};
+}
+
 // The host checks of launch_select alone, nothing enqueued: a multi-launch
 // entry point runs them before its first launch, so an argument error leaves
 // every output untouched.
@@ -2349,18 +2624,14 @@ int launch_attention_then_count(const float* q, const uint8_t* k_pool, const uin
     const dim3 grid(32 * 4 + groups * js.count);
     const float* part = static_cast<const float*>(workspace);
     const bool wide = b.count_width() == kWideCount;
-    if (b.any_current && wide)
-        hipLaunchKernelGGL((combine_count_kernel<true, kWideCount>), grid, dim3(kThreads), 0,
-                           stream, part, chunks, out, js, groups);
-    else if (b.any_current)
-        hipLaunchKernelGGL((combine_count_kernel<true, 1>), grid, dim3(kThreads), 0, stream, part,
-                           chunks, out, js, groups);
-    else if (wide)
-        hipLaunchKernelGGL((combine_count_kernel<false, kWideCount>), grid, dim3(kThreads), 0,
-                           stream, part, chunks, out, js, groups);
-    else
-        hipLaunchKernelGGL((combine_count_kernel<false, 1>), grid, dim3(kThreads), 0, stream, part,
-                           chunks, out, js, groups);
+    const auto kernel =
+        b.any_current ? (wide            ? combine_count_kernel<true, kWideCount, true>
+                         : b.all_aligned ? combine_count_kernel<true, 1, true>
+                                         : combine_count_kernel<true, 1, false>)
+                      : (wide            ? combine_count_kernel<false, kWideCount, true>
+                         : b.all_aligned ? combine_count_kernel<false, 1, true>
+                                         : combine_count_kernel<false, 1, false>);
+    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, part, chunks, out, js, groups);
     const hipError_t st = hipGetLastError();
     return st == hipSuccess ? HS_OK : hip_fail(st, "attention-then-count launch");
 }
