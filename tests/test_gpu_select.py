@@ -446,3 +446,24 @@ def test_mixed_word_counts_in_a_batch(hs, port):
                 assert rc == 0 and st["code"] == 0 and st["k"] == k and st["boundary_tied_heads"] == tied
                 assert np.array_equal(from_dev(counts), pcounts)
                 assert np.array_equal(from_dev(ids)[:, :k], np.sort(pids, axis=1) if id_order else pids)
+
+
+@pytest.mark.parametrize("offset", range(8))
+def test_rows_off_sixteen_bytes(hs, port, offset):
+    # score rows at every offset within 16 bytes (an odd stride, a base off by
+    # 0..7 ids): the count reads two aligned words per 8 ids and moves them
+    # down; the first and last ids of the scores are read one by one
+    g = rng(60 + offset)
+    for n, stride in ((8, 9), (4097, 4099), (9001, 9003)):
+        s = f16_bits(g.standard_normal((8, stride)) * 3.0)
+        s[0, 0] = s[7, n - 1] = hb(11.0)  # both ends are selected
+        flat = np.concatenate([np.full(offset, hb(60000), dtype=np.uint16), s.reshape(-1)[: 7 * stride + n]])
+        rc, k, ids, counts, tied = port.select(s, 8, stride, n, 4.0, 0.5)
+        dev = to_dev(flat)[offset:]
+        assert dev.data_ptr() % 16 == 2 * offset
+        for id_order in (False, True):
+            got, gcounts, _, status = hs.ops.select(dev, 8, stride, n, 4.0, 0.5, id_order=id_order)
+            st = hs.ops.read_status(status)
+            assert st["code"] == rc == 0 and st["k"] == k and st["boundary_tied_heads"] == tied
+            assert np.array_equal(from_dev(gcounts), counts)
+            assert np.array_equal(from_dev(got)[:, :k], np.sort(ids, axis=1) if id_order else ids)
