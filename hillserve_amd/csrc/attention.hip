@@ -13,8 +13,8 @@
 // whose mask entry is 0.  FP32 accumulation, FP32 softmax.
 //
 // Work split (flash-decoding over the token axis):
-//  * grid (chunks); a workgroup owns 128 token ids and all 8 KV heads, one
-//    wave per KV head g.  A wave ORs its 4 query heads' selection bitmaps,
+//  * grid (chunks); a workgroup owns 32, 64 or 128 token ids (attn_chunk) and
+//    all 8 KV heads, one wave per KV head g.  A wave ORs its 4 query heads' selection bitmaps,
 //    compacts the union in id order, and reads each selected (id, g) K row
 //    and V row exactly once for all of its query heads -> HBM bytes =
 //    sum_g |U_g|*512.  The 8 waves read the 8 heads' segments of the same
@@ -40,7 +40,6 @@
 namespace hs {
 namespace {
 
-constexpr uint32_t kChunk = kAttnChunk;  // token ids per workgroup
 constexpr uint32_t kThreads = 512; // 8 waves: one per KV head
 constexpr uint32_t kRecord = kAttnRecord;
 constexpr float kScale = 0.088388347648318440550f;  // 1/sqrt(128)
@@ -105,7 +104,7 @@ __device__ __forceinline__ void accumulate_pair(float (&o)[4][8], const half2v (
 // 364.7 us against 368.0; no difference at 24576 and below, where the V rows
 // of a pass may come from the caches themselves.
 constexpr uint32_t kStreamTokens = 28672;
-template <bool kRows, bool kStream>
+template <bool kRows, bool kStream, uint32_t kChunk>
 __global__ void __launch_bounds__(kThreads)
 attn_kv_kernel(const float* __restrict__ q, const uint8_t* __restrict__ pool, uint32_t row_bytes,
                int64_t v_delta, const int32_t* __restrict__ rows, uint32_t pool_rows,
@@ -120,7 +119,7 @@ attn_kv_kernel(const float* __restrict__ q, const uint8_t* __restrict__ pool, ui
     const uint32_t g = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave = KV head
     const uint32_t words = (n + 31) / 32, base = chunk * kChunk;
     const uint32_t r16 = lane & 15u, q16 = lane >> 4;
-    constexpr uint32_t kSteps = kChunk / 64;
+    constexpr uint32_t kSteps = (kChunk + 63) / 64;  // (32 ids: the upper lanes hold none)
     uint32_t mw[kSteps][4];
 #pragma unroll
     for (uint32_t c = 0; c < kSteps; ++c) {
@@ -133,7 +132,7 @@ attn_kv_kernel(const float* __restrict__ q, const uint8_t* __restrict__ pool, ui
     for (uint32_t c = 0; c < kSteps; ++c) {
         const uint32_t id = base + 64 * c + lane;
         uint32_t mk = 0, r = id;
-        if (id < n) {
+        if (id < n && (kChunk >= 64 || lane < kChunk)) {
 #pragma unroll
             for (uint32_t j = 0; j < 4; ++j) mk |= ((mw[c][j] >> (id & 31u)) & 1u) << j;
             if (kRows && mk) {
@@ -259,7 +258,8 @@ attn_kv_kernel(const float* __restrict__ q, const uint8_t* __restrict__ pool, ui
                 p[j] = sv[j] == -INFINITY ? 0.0f : weight_f16(__expf(sv[j] - m[j]));
                 ps[j] += p[j];
             }
-            sel_p[g][64 * c + lane] = make_float4(p[0], p[1], p[2], p[3]);  // 0 past the union
+            if (kChunk >= 64 || lane < kChunk)
+                sel_p[g][64 * c + lane] = make_float4(p[0], p[1], p[2], p[3]);  // 0 past the union
         }
 #pragma unroll
         for (uint32_t j = 0; j < 4; ++j) lsum[j] = first_lane(wave_sum_f32(ps[j]));
@@ -323,7 +323,7 @@ attn_kv_kernel(const float* __restrict__ q, const uint8_t* __restrict__ pool, ui
 constexpr uint32_t kBufferLimit = 0xffff0000u, kPastEnd = 0xfffffff0u;
 constexpr int kBufferWord3 = 0x00020000;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-template <bool kRows, bool kBuffer>
+template <bool kRows, bool kBuffer, uint32_t kChunk>
 __global__ void __launch_bounds__(kThreads)
 attn_v_kernel(const float* __restrict__ dots, uint32_t dstride, const uint8_t* __restrict__ v_pool,
               uint32_t row_bytes, const int32_t* __restrict__ rows, uint32_t pool_rows,
@@ -336,7 +336,7 @@ attn_v_kernel(const float* __restrict__ dots, uint32_t dstride, const uint8_t* _
     const uint32_t chunk = blockIdx.x, tid = threadIdx.x, lane = tid & 63u;
     const uint32_t g = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave = KV head
     const uint32_t words = (n + 31) / 32, base = chunk * kChunk;
-    constexpr uint32_t kSteps = kChunk / 64;
+    constexpr uint32_t kSteps = (kChunk + 63) / 64;  // (32 ids: the upper lanes hold none)
     uint32_t mw[kSteps][4];
     float sd[kSteps][4];
 #pragma unroll
@@ -353,7 +353,7 @@ attn_v_kernel(const float* __restrict__ dots, uint32_t dstride, const uint8_t* _
     for (uint32_t c = 0; c < kSteps; ++c) {
         const uint32_t id = base + 64 * c + lane;
         uint32_t mk = 0, r = id;
-        if (id < n) {
+        if (id < n && (kChunk >= 64 || lane < kChunk)) {
 #pragma unroll
             for (uint32_t j = 0; j < 4; ++j) mk |= ((mw[c][j] >> (id & 31u)) & 1u) << j;
             if (kRows && mk) {
@@ -464,7 +464,8 @@ attn_v_kernel(const float* __restrict__ dots, uint32_t dstride, const uint8_t* _
                 p[j] = sv[j] == -INFINITY ? 0.0f : weight_f16(__expf(sv[j] - m[j]));
                 ps[j] += p[j];
             }
-            sel_p[g][64 * c + lane] = make_float4(p[0], p[1], p[2], p[3]);  // 0 past the union
+            if (kChunk >= 64 || lane < kChunk)
+                sel_p[g][64 * c + lane] = make_float4(p[0], p[1], p[2], p[3]);  // 0 past the union
         }
 #pragma unroll
         for (uint32_t j = 0; j < 4; ++j) lsum[j] = first_lane(wave_sum_f32(ps[j]));
@@ -515,8 +516,12 @@ attn_combine_kernel(const float* __restrict__ part, uint32_t chunks, float* __re
 }  // namespace
 
 size_t attention_workspace_bytes(uint32_t n) {
-    const size_t chunks = (static_cast<size_t>(n) + kChunk - 1) / kChunk;
-    return align256(sizeof(float) * 8 * chunks * 4 * kRecord);
+    // not smaller for more tokens, though their chunks are longer: a workspace
+    // sized for the longest sequence serves every shorter one
+    uint32_t chunks = attn_chunks(n);
+    for (const uint32_t line : {kAttnShort, kAttnMiddle})
+        if (n > line) chunks = std::max(chunks, attn_chunks(line));
+    return align256(sizeof(float) * 8 * size_t(chunks) * 4 * kRecord);
 }
 
 int launch_attention_partial(const float* q, const uint8_t* k_pool, const uint8_t* v_pool,
@@ -531,11 +536,18 @@ int launch_attention_partial(const float* q, const uint8_t* k_pool, const uint8_
     if ((reinterpret_cast<uintptr_t>(k_pool) | reinterpret_cast<uintptr_t>(v_pool)) & 15u)
         return reject("attention: K and V pools must be 16-byte aligned");
     const int64_t v_delta = reinterpret_cast<intptr_t>(v_pool) - reinterpret_cast<intptr_t>(k_pool);
-    const uint32_t chunks = (n + kChunk - 1) / kChunk;
+    const uint32_t chunks = attn_chunks(n);
     float* part = static_cast<float*>(workspace);
     const bool streamed = n >= kStreamTokens;
-    const auto kernel = rows ? (streamed ? attn_kv_kernel<true, true> : attn_kv_kernel<true, false>)
-                             : (streamed ? attn_kv_kernel<false, true> : attn_kv_kernel<false, false>);
+    const auto kernel = [&] {
+        switch (attn_chunk(n)) {
+        case 32: return rows ? attn_kv_kernel<true, false, 32> : attn_kv_kernel<false, false, 32>;
+        case 64: return rows ? attn_kv_kernel<true, false, 64> : attn_kv_kernel<false, false, 64>;
+        default:
+            return rows ? (streamed ? attn_kv_kernel<true, true, kAttnChunk> : attn_kv_kernel<true, false, kAttnChunk>)
+                        : (streamed ? attn_kv_kernel<false, true, kAttnChunk> : attn_kv_kernel<false, false, kAttnChunk>);
+        }
+    }();
     hipLaunchKernelGGL(kernel, dim3(chunks), dim3(kThreads), 0, stream, q, k_pool,
                        static_cast<uint32_t>(row_bytes), v_delta, rows, rows ? pool_rows : 0u,
                        member, n, chunks, part);
@@ -555,28 +567,29 @@ int launch_attention_logits(const float* logits, size_t logit_stride, const uint
     if (row_bytes < 2048 || row_bytes % 16 != 0 || row_bytes > (1u << 20))
         return reject("attention: row_bytes must be 2048..1 MiB and a multiple of 16");
     if (reinterpret_cast<uintptr_t>(v_pool) & 15u) return reject("attention: V pool must be 16-byte aligned");
-    const uint32_t chunks = (n + kChunk - 1) / kChunk;
+    const uint32_t chunks = attn_chunks(n);
     float* part = static_cast<float*>(workspace);
     const auto ls = static_cast<uint32_t>(logit_stride);
     const auto rb = static_cast<uint32_t>(row_bytes);
     // the rows a V read can reach: the pool's rows, or ids below n
     const uint64_t pool_bytes = static_cast<uint64_t>(rows ? pool_rows : n) * row_bytes;
-    const auto pb = static_cast<uint32_t>(pool_bytes);
-    if (pool_bytes < kBufferLimit) {
-        if (rows)
-            hipLaunchKernelGGL((attn_v_kernel<true, true>), dim3(chunks), dim3(kThreads), 0, stream, logits,
-                               ls, v_pool, rb, rows, pool_rows, pb, member, n, chunks, part);
-        else
-            hipLaunchKernelGGL((attn_v_kernel<false, true>), dim3(chunks), dim3(kThreads), 0, stream, logits,
-                               ls, v_pool, rb, rows, 0u, pb, member, n, chunks, part);
-    } else {
-        if (rows)
-            hipLaunchKernelGGL((attn_v_kernel<true, false>), dim3(chunks), dim3(kThreads), 0, stream, logits,
-                               ls, v_pool, rb, rows, pool_rows, 0u, member, n, chunks, part);
-        else
-            hipLaunchKernelGGL((attn_v_kernel<false, false>), dim3(chunks), dim3(kThreads), 0, stream, logits,
-                               ls, v_pool, rb, rows, 0u, 0u, member, n, chunks, part);
-    }
+    const bool buffer = pool_bytes < kBufferLimit;
+    const auto kernel = [&] {
+        switch (attn_chunk(n)) {
+        case 32:
+            return rows ? (buffer ? attn_v_kernel<true, true, 32> : attn_v_kernel<true, false, 32>)
+                        : (buffer ? attn_v_kernel<false, true, 32> : attn_v_kernel<false, false, 32>);
+        case 64:
+            return rows ? (buffer ? attn_v_kernel<true, true, 64> : attn_v_kernel<true, false, 64>)
+                        : (buffer ? attn_v_kernel<false, true, 64> : attn_v_kernel<false, false, 64>);
+        default:
+            return rows ? (buffer ? attn_v_kernel<true, true, kAttnChunk> : attn_v_kernel<true, false, kAttnChunk>)
+                        : (buffer ? attn_v_kernel<false, true, kAttnChunk> : attn_v_kernel<false, false, kAttnChunk>);
+        }
+    }();
+    hipLaunchKernelGGL(kernel, dim3(chunks), dim3(kThreads), 0, stream, logits, ls, v_pool, rb, rows,
+                       rows ? pool_rows : 0u, buffer ? static_cast<uint32_t>(pool_bytes) : 0u, member, n,
+                       chunks, part);
     hipLaunchKernelGGL(attn_combine_kernel, dim3(32, 4), dim3(kCombineThreads), 0, stream,
                        static_cast<const float*>(workspace), chunks, out);
     const hipError_t st = hipGetLastError();
@@ -590,7 +603,7 @@ int launch_attention(const float* q, const uint8_t* k_pool, const uint8_t* v_poo
     const int rc = launch_attention_partial(q, k_pool, v_pool, row_bytes, rows, pool_rows, member,
                                             n, out, workspace, stream);
     if (rc != HS_OK) return rc;
-    const uint32_t chunks = (n + kChunk - 1) / kChunk;
+    const uint32_t chunks = attn_chunks(n);
     hipLaunchKernelGGL(attn_combine_kernel, dim3(32, 4), dim3(kCombineThreads), 0, stream,
                        static_cast<const float*>(workspace), chunks, out);
     const hipError_t st = hipGetLastError();

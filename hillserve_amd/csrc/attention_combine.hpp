@@ -12,7 +12,18 @@
 
 namespace hs {
 
-constexpr uint32_t kAttnChunk = 128;      // token ids per partial workgroup
+// Token ids per partial workgroup: the shortest of 32, 64 and 128 that makes at
+// most 256 workgroups, one for each CU.  A workgroup is a chain of round trips
+// (membership, rows, record), and 128 ids on a quarter of the CUs make each
+// of its steps longer than it need be.  Eight pipelined layers of 2048 / 8192
+// / 16384 tokens take 226 / 255 / 290 us against 275 / 297 / 321 with 128 ids
+// everywhere, one layer (V rows only) of 3001 / 8192 / 16384 23.0 / 26.4 /
+// 32.7 against 24.9 / 28.0 / 33.8.  More workgroups than CUs do not pay: 32 ids
+// at 16384 tokens 35.2 us, 64 at 32768 45.1 against 43.8, twice the records.
+constexpr uint32_t kAttnChunk = 128;
+constexpr uint32_t kAttnShort = 256 * 32, kAttnMiddle = 256 * 64;
+inline uint32_t attn_chunk(uint32_t n) { return n <= kAttnShort ? 32u : n <= kAttnMiddle ? 64u : kAttnChunk; }
+inline uint32_t attn_chunks(uint32_t n) { return (n + attn_chunk(n) - 1) / attn_chunk(n); }
 constexpr uint32_t kAttnRecord = 2 + 128;  // m, l, o[128] per (chunk, query head)
 
 // Merge the per-chunk (m, l, o) records of query head h, channels
@@ -94,7 +105,7 @@ __device__ __forceinline__ void combine_batch(const float* __restrict__ part, ui
 }
 
 // The batch is chosen by the number of chunks: 4, 16 or 32 values per thread
-// for n <= 8192, 32768 and 65536 (the order of the sum does not depend on
+// for up to 64, 256 and 512 of them (the order of the sum does not depend on
 // it).  A batch whose later values were read one by
 // one in a loop made n = 65536 wait a round trip per 16 chunks: its layer
 // takes 72.8 us with 32 values at once against 77.6.  The short batch takes

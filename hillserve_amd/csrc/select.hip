@@ -2632,7 +2632,7 @@ int launch_attention_then_count(const float* q, const uint8_t* k_pool, const uin
     if (rc != HS_OK) return rc;
     // the merge reads the attention records and writes out while the count
     // reads the next scores and writes its workspace and status
-    const uint32_t chunks = (n + kAttnChunk - 1) / kAttnChunk;
+    const uint32_t chunks = attn_chunks(n);
     const Span merge_in = span(workspace, sizeof(float) * 8 * size_t(chunks) * 4 * kAttnRecord);
     const Span merge_out = span(out, sizeof(float) * 32 * 128);
     for (uint32_t j = 0; j < next_count; ++j) {

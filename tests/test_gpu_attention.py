@@ -190,3 +190,33 @@ def test_merge_batches_and_streamed_rows(hs, port, n):
                                   to_dev(member_words(ids, n).reshape(-1)))
     ref = port.attention(q, pool.view(np.uint8), ids)
     assert rel_err(out.cpu().numpy().astype(np.float64), ref) <= TOL
+
+
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 65, 8191, 8192, 8193, 16384, 16385])
+def test_chunk_lengths(hs, port, n):
+    # chunks of 32 ids up to 8192 tokens, 64 up to 16384, 128 beyond: full
+    # and ragged last chunks with almost every row selected, K and V rows
+    # and V rows with the scoring pass's dots
+    g = rng(40 + n)
+    k = f16_bits(g.standard_normal((n, 8, 128)))
+    v = f16_bits(g.standard_normal((n, 8, 128)))
+    pool = pool_rows(k, v)
+    q = g.standard_normal((32, 128)).astype(np.float32)
+    ids = [np.flatnonzero((g.random(n) < 0.95) | (np.arange(n) == n - 1)) for _ in range(32)]
+    member = to_dev(member_words(ids, n).reshape(-1))
+    qd = torch.from_numpy(q).cuda()
+    out = hs.ops.sparse_attention(qd, to_dev(pool.reshape(-1)), n, member)
+    ref = port.attention(q, pool.view(np.uint8), ids)
+    assert rel_err(out.cpu().numpy().astype(np.float64), ref) <= TOL
+    _, dots = hs.ops.score_logits(to_dev(f16_bits(q).reshape(-1)), qd, to_dev(k.reshape(-1)), n)
+    out = hs.ops.sparse_attention_logits(dots, to_dev(v.reshape(-1)), n, member)
+    assert rel_err(out.cpu().numpy().astype(np.float64), ref) <= TOL
+
+
+def test_workspace_of_longer_sequences_serves_shorter(hs):
+    size = hs.lib().hs_gqa_attention_workspace_bytes
+    layer = hs.lib().hs_decode_layer_workspace_bytes
+    ns = sorted({1, 65536, *range(500, 65536, 977), *(x + d for x in (8192, 16384, 32768) for d in (-1, 0, 1))})
+    for f in (size, layer):
+        got = [f(n) for n in ns]
+        assert got == sorted(got)
