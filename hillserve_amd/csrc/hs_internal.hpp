@@ -40,6 +40,8 @@ inline hipStream_t as_stream(void* stream) { return static_cast<hipStream_t>(str
 // Round a byte count up to 256 B so workspace slices stay aligned.
 inline size_t align256(size_t bytes) { return (bytes + 255) & ~size_t(255); }
 
+// hs_decode_layer: up to so many tokens one launch counts and selects.
+constexpr uint32_t kShortTokens = 8192;
 // Words that hs_decode_layer's scoring launch clears for the selection that
 // follows it: 32 published counts, 32 tie records of 8 bytes and the status's
 // tied-head count (all null: nothing to clear).

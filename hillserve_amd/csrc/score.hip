@@ -71,19 +71,48 @@ score_kernel(const ScoreJobs jobs, const int32_t* __restrict__ rows, uint32_t po
 template <bool kRows, bool kStream>
 __global__ void __launch_bounds__(kWavesPerBlock * 64) __attribute__((amdgpu_waves_per_eu(4)))
 score_logits_kernel(const ScoreJobs jobs, const int32_t* __restrict__ rows, uint32_t pool_rows,
-                    const LogitsOut lo, const SelectExchange clear) {
-    if (!kStream && clear.published && blockIdx.x == 0) {  // for the selection that follows
-        const uint32_t tid = threadIdx.x;
-        if (tid < 32) clear.published[tid] = 0;
-        if (tid < 64) clear.ties[tid] = 0;
-        if (tid == 0) *clear.tied_heads = 0;
-    }
+                    const LogitsOut lo) {
     __shared__ uint4 lds[kWavesPerBlock][kHalfTileChunks];
     __shared__ uint4 qstage[kWavesPerBlock][8 * 16];
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     score_waves<kRows, false, true, kStream>(
         jobs, rows, pool_rows, __builtin_amdgcn_readfirstlane(blockIdx.x * kWavesPerBlock + w),
         gridDim.x * kWavesPerBlock, lds[w], lo, qstage[w]);
+}
+
+// Up to kShortIds (token tile, KV head) pairs, four per CU: a wave of its own
+// workgroup for each, spread over all CUs, both halves of its tile in flight
+// at once (in two-wave workgroups half the CUs would hold two waves, and
+// the second half waits for the first).  One layer of 1024 tokens 19.6 -> 19.1
+// us, of 7919 in 4096 B records 27.4 -> 26.9, of 8192 26.4 -> 24.8; score, cover
+// and union of 1024 24.4 -> 24.1.  From 12288 tokens on the waves fill the CUs
+// and it is slower (30.8 -> 31.5 us a layer).
+constexpr uint32_t kShortIds = 1024;
+static_assert(kShortIds >= kShortTokens / kTileTokens * 8, "the launches that clear the exchange words");
+
+// By one wave of the launch before launch_layer_select.
+__device__ __forceinline__ void clear_exchange(const SelectExchange& clear) {
+    const uint32_t lane = threadIdx.x & 63u;
+    if (clear.published == nullptr) return;
+    if (lane < 32) clear.published[lane] = 0;
+    clear.ties[lane] = 0;
+    if (lane == 0) *clear.tied_heads = 0;
+}
+
+template <bool kRows, bool kBatch>
+__global__ void __launch_bounds__(64)
+score_short_kernel(const ScoreJobs jobs, const int32_t* __restrict__ rows, uint32_t pool_rows) {
+    __shared__ uint4 lds[kHalfTileChunks];
+    score_waves<kRows, kBatch, false, false, true>(jobs, rows, pool_rows, blockIdx.x, gridDim.x, lds);
+}
+template <bool kRows>
+__global__ void __launch_bounds__(64)
+score_logits_short_kernel(const ScoreJobs jobs, const int32_t* __restrict__ rows, uint32_t pool_rows,
+                          const LogitsOut lo, const SelectExchange clear) {
+    if (blockIdx.x == 0) clear_exchange(clear);
+    __shared__ uint4 lds[kHalfTileChunks];
+    __shared__ uint4 qstage[8 * 16];
+    score_waves<kRows, false, true, false, true>(jobs, rows, pool_rows, blockIdx.x, gridDim.x, lds, lo, qstage);
 }
 
 // 16 waves per CU (four per SIMD, 8 KiB of LDS each), each streaming its
@@ -124,13 +153,23 @@ int launch_score(const uint16_t* q, const uint16_t* keys, size_t stride_words,
     const LogitsOut lo{qf, logits, static_cast<uint32_t>(logit_stride), vec};
     jobs.total_ids = ((tokens + kTileTokens - 1) / kTileTokens) * 8;  // (token tile, KV head)
     const dim3 grid(score_grid(jobs.total_ids)), block(kWavesPerBlock * 64);
+    if (jobs.total_ids <= kShortIds) {
+        const dim3 short_grid(jobs.total_ids), wave(64);
+        if (logits)
+            hipLaunchKernelGGL((rows ? score_logits_short_kernel<true> : score_logits_short_kernel<false>),
+                               short_grid, wave, 0, stream, jobs, rows, rows ? pool_rows : 0u, lo, clear);
+        else
+            hipLaunchKernelGGL((rows ? score_short_kernel<true, false> : score_short_kernel<false, false>),
+                               short_grid, wave, 0, stream, jobs, rows, rows ? pool_rows : 0u);
+        const hipError_t status = hipGetLastError();
+        return status == hipSuccess ? HS_OK : hip_fail(status, "score launch");
+    }
     const uint64_t key_bytes = uint64_t(tokens) * 2048;
     const bool streamed = key_bytes >= (logits ? kStreamLogitKeyBytes : kStreamKeyBytes);
     if (logits) {
         const auto kernel = rows ? (streamed ? score_logits_kernel<true, true> : score_logits_kernel<true, false>)
                                  : (streamed ? score_logits_kernel<false, true> : score_logits_kernel<false, false>);
-        hipLaunchKernelGGL(kernel, grid, block, 0, stream, jobs, rows, rows ? pool_rows : 0u, lo,
-                           clear);
+        hipLaunchKernelGGL(kernel, grid, block, 0, stream, jobs, rows, rows ? pool_rows : 0u, lo);
     } else {
         const auto kernel = rows ? (streamed ? score_kernel<true, false, true> : score_kernel<true, false, false>)
                                  : (streamed ? score_kernel<false, false, true> : score_kernel<false, false, false>);
@@ -169,10 +208,15 @@ int launch_score_batched(const hs_score_job_t* jobs, uint32_t count, hipStream_t
     if (rc != HS_OK) return rc;
     uint64_t key_bytes = 0;
     for (uint32_t i = 0; i < count; ++i) key_bytes += uint64_t(jobs[i].tokens) * 2048;
-    const auto kernel = key_bytes >= kStreamKeyBytes ? score_kernel<false, true, true>
-                                                     : score_kernel<false, true, false>;
-    hipLaunchKernelGGL(kernel, dim3(score_grid(table.total_ids)), dim3(kWavesPerBlock * 64), 0,
-                       stream, table, nullptr, 0u);
+    if (table.total_ids <= kShortIds) {
+        hipLaunchKernelGGL((score_short_kernel<false, true>), dim3(table.total_ids), dim3(64), 0, stream,
+                           table, nullptr, 0u);
+    } else {
+        const auto kernel = key_bytes >= kStreamKeyBytes ? score_kernel<false, true, true>
+                                                         : score_kernel<false, true, false>;
+        hipLaunchKernelGGL(kernel, dim3(score_grid(table.total_ids)), dim3(kWavesPerBlock * 64), 0,
+                           stream, table, nullptr, 0u);
+    }
     const hipError_t status = hipGetLastError();
     return status == hipSuccess ? HS_OK : hip_fail(status, "score batch launch");
 }

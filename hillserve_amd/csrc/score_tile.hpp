@@ -53,7 +53,8 @@ int build_score_jobs(const hs_score_job_t* jobs, uint32_t count, ScoreJobs& out)
 // wave, wave + waves, ... of `jobs`; `region` is its own kHalfTileChunks
 // of LDS.  Waves never wait on one another.  A tile's second half is
 // requested once its first is parked in LDS, into the same registers.
-// (Both halves requested together cost 32 more VGPRs and measured slower.)
+// (Both halves requested together cost 32 more VGPRs and measured slower
+// wherever the chip is full; kOneTile does it below that.)
 // kLogits: the same pass also produces the attention's q.k dots of the
 // tile's 64 tokens for the 4 query heads (F32 queries lo.qf), on MFMA from
 // the K values the ordered chains already hold: v_mfma_f32_4x4x4_16b_f16
@@ -66,8 +67,9 @@ int build_score_jobs(const hs_score_job_t* jobs, uint32_t count, ScoreJobs& out)
 // head j's dots of tokens 4b .. 4b+3, written to lo.out unscaled; the
 // attention then reads V rows only.
 // kStream: the keys are read with the nontemporal hint (the launches decide,
-// score.hip).
-template <bool kRows, bool kBatch, bool kLogits = false, bool kStream = false>
+// score.hip).  kOneTile: as many waves as ids; a wave requests both halves of
+// its only tile at once.
+template <bool kRows, bool kBatch, bool kLogits = false, bool kStream = false, bool kOneTile = false>
 __device__ __forceinline__ void score_waves(const ScoreJobs& jobs, const int32_t* __restrict__ rows,
                                             uint32_t pool_rows, uint32_t wave, uint32_t waves,
                                             uint4* region, const LogitsOut& lo = LogitsOut{},
@@ -270,6 +272,20 @@ __device__ __forceinline__ void score_waves(const ScoreJobs& jobs, const int32_t
     ScoreJob cur = jobs.job[job_of(id)];
     uint32_t row = row_of(cur, id);
     load(cur, id, 0, row, v);
+    if constexpr (kOneTile) {
+        uint4 second[kHalf];
+        load(cur, id, 1, row, second);
+        if constexpr (kLogits) stage_query((id - cur.first_id) & 7u);
+        stash(v);
+        __builtin_amdgcn_wave_barrier();
+        compute(cur, id, 0);
+        __builtin_amdgcn_wave_barrier();
+        stash(second);
+        __builtin_amdgcn_wave_barrier();
+        compute(cur, id, 1);
+        finish(cur, id);
+        return;
+    }
     while (true) {
         if constexpr (kLogits) {
             const uint32_t kv = (id - cur.first_id) & 7u;  // wave-uniform

@@ -1809,7 +1809,7 @@ __global__ void __launch_bounds__(kHThreads) head_select_kernel(const SelectJobs
 // tokens takes 22.2 us against 27.8, of 4096 23.8 against 28.5, of 8192 28.1
 // against 31.7.  At 16384 ids (512 threads of 32) it gained 0.7 us and at 12288
 // it lost 0.6, so the line is 8192.
-constexpr uint32_t kSmallMaxN = 8192;
+constexpr uint32_t kSmallMaxN = kShortTokens;
 constexpr uint32_t kPublished = 0x80000000u, kPublishedBad = 0x40000000u;
 
 __device__ __forceinline__ uint64_t realtime_ticks() { return __builtin_amdgcn_s_memrealtime(); }

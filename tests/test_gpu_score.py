@@ -119,3 +119,26 @@ def test_head0_partial_maxima(hs, port):
     keys = np.array([port.order_key(int(b)) for b in raw[0]])
     expected = [keys[i * 64:(i + 1) * 64].max() for i in range((n + 63) // 64)]
     assert np.array_equal(from_dev(partial), np.array(expected, dtype=np.uint32))
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 8128, 8192, 8193])
+def test_one_wave_per_tile(hs, port, n):
+    # up to 8192 tokens every (token tile, KV head) pair has a wave of its own
+    # that requests both halves of its tile at once: single and batched,
+    # plain and with the attention's dots, with a row map
+    g = rng(30 + n)
+    q, k = mixed_finite(g, (32, 128)), mixed_finite(g, (n, 8, 128))
+    want = port.score(q, k.reshape(-1), n, 1024)
+    part = torch.zeros((n + 63) // 64, dtype=torch.int32, device="cuda")
+    assert np.array_equal(from_dev(hs.ops.score(to_dev(q.reshape(-1)), to_dev(k.reshape(-1)), n, head0_partial=part)), want)
+    perm = g.permutation(n).astype(np.int32)
+    mapped = to_dev(k[np.argsort(perm)].reshape(-1))
+    part2 = torch.zeros_like(part)
+    raw, _ = hs.ops.score_logits(to_dev(q.reshape(-1)), torch.zeros((32, 128), device="cuda"), mapped, n,
+                                 rows=to_dev(perm), head0_partial=part2)
+    assert np.array_equal(from_dev(raw), want) and torch.equal(part, part2)
+    assert np.array_equal(from_dev(hs.ops.score(to_dev(q.reshape(-1)), mapped, n, rows=to_dev(perm))), want)
+    cut = n // 3
+    jobs = [dict(q16=to_dev(q.reshape(-1)), keys=to_dev(k[a:b].reshape(-1)), tokens=b - a)
+            for a, b in ((0, cut), (cut, n)) if b > a]
+    assert np.array_equal(np.concatenate([from_dev(x) for x in hs.ops.score_batched(jobs)], axis=1), want)
