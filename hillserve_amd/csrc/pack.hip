@@ -181,7 +181,12 @@ __device__ __forceinline__ const uint8_t* fallback_row(const PoolSource& ps, con
     return nullptr;
 }
 
-// Grid (ceil(count/64), 32 heads), 256 threads.  kPack selects the source.
+// Grid (ceil(count/kSlots), 32 heads), 4 threads per slot.  kPack selects the
+// source.  64 slots at a time; 32 up to kShortSlots, where 64 would leave the
+// chip's 8 workgroups per CU unfilled (gather of 1664 slots 10.6 -> 9.4 us, pack
+// of 3296 slots with its union 28.8 -> 28.0) and above which the shorter runs of
+// V cost more than the finer split gives (6560 slots: gather 43.5 -> 44.8, pack
+// 59.6 -> 62.2).
 // Bound by HBM: at 6560 slots the pack moves 269 MB (161 MB written), the
 // gather 215 MB (107 MB written).  The packed K, V and mask leave through
 // streaming stores: nothing here reads them back, and through the ordinary
@@ -191,17 +196,20 @@ __device__ __forceinline__ const uint8_t* fallback_row(const PoolSource& ps, con
 // 73.7 us; 3296 slots, 49.1 -> 37.6 us; gather of 6560 slots 45.6 -> 43.6 us,
 // of 1664 slots 11.6 -> 10.6 us.  (Streaming loads of the rows as well lose
 // that reuse: 76.3, 45.3, 44.5 and 13.4 us.)
-template <bool kPack>
-__global__ void __launch_bounds__(256)
+constexpr uint32_t kShortSlots = 256 * 8 / 32 * 64;
+template <bool kPack, uint32_t kSlots>
+__global__ void __launch_bounds__(kSlots * 4)
 pack_kernel(PoolSource ps, MapSource ms, const uint64_t* __restrict__ positions, uint32_t nq,
             uint32_t count, uint16_t* __restrict__ k_out, uint16_t* __restrict__ v_out,
             float* __restrict__ mask, hs_status_t* __restrict__ status, uint32_t stamp) {
-    __shared__ uint4 vtile[64][17];  // 64 slots x 256 B V half row (+pad)
-    __shared__ const uint8_t* src_row[64];
-    __shared__ uint32_t slot_id[64], slot_ok[64];
-    const uint32_t h = blockIdx.y, kv = h >> 2, s0 = blockIdx.x * 64, tid = threadIdx.x;
+    constexpr uint32_t kT = kSlots * 4;
+    static_assert(kSlots <= 64 && kSlots % 8 == 0, "one wave looks the slots up");
+    __shared__ uint4 vtile[kSlots][17];  // kSlots x 256 B V half row (+pad)
+    __shared__ const uint8_t* src_row[kSlots];
+    __shared__ uint32_t slot_id[kSlots], slot_ok[kSlots];
+    const uint32_t h = blockIdx.y, kv = h >> 2, s0 = blockIdx.x * kSlots, tid = threadIdx.x;
 
-    if (tid < 64) {  // wave 0
+    if (tid < kSlots) {  // wave 0
         const uint32_t s = s0 + tid;
         const uint8_t* src = nullptr;
         uint32_t id = 0xffffffffu;
@@ -255,7 +263,7 @@ pack_kernel(PoolSource ps, MapSource ms, const uint64_t* __restrict__ positions,
         if (tid == 0) publish_stamped(status, stamp, first, blockIdx.x == 0 && blockIdx.y == 0);
     }
     __syncthreads();
-    // K rows: 64 slots x 16 x 16 B; V half rows staged for the transpose.
+    // K rows: kSlots x 16 x 16 B; V half rows staged for the transpose.
     // (prefetched and miss rows are 4096 B records: V 2048 B after K)
     const int64_t v_delta = kPack ? ps.v_delta : 2048;
     // Every K and V chunk of the thread's 4 (slot, chunk) pairs is requested
@@ -264,12 +272,12 @@ pack_kernel(PoolSource ps, MapSource ms, const uint64_t* __restrict__ positions,
     // can only be waited for all at once).  With no source at all (every
     // slot empty) nothing is read.
     using GlobalU32 = const __attribute__((address_space(1))) uint32_t;
-    constexpr uint32_t kPairs = 64 * 16 / 256;
+    constexpr uint32_t kPairs = kSlots * 16 / kT;
     uint4 kw[kPairs], vw[kPairs];
     if (fallback_row(ps, ms, kPack) != nullptr) {
 #pragma unroll
         for (uint32_t u = 0; u < kPairs; ++u) {
-            const uint32_t i = tid + 256 * u, s = i >> 4, c = i & 15u;
+            const uint32_t i = tid + kT * u, s = i >> 4, c = i & 15u;
             const uint8_t* src = src_row[s];
             GlobalU32* kp = (GlobalU32*)(src + kv * 256) + 4 * c;
             GlobalU32* vp = (GlobalU32*)(src + v_delta + kv * 256) + 4 * c;
@@ -282,7 +290,7 @@ pack_kernel(PoolSource ps, MapSource ms, const uint64_t* __restrict__ positions,
     }
 #pragma unroll
     for (uint32_t u = 0; u < kPairs; ++u) {
-        const uint32_t i = tid + 256 * u, s = i >> 4, c = i & 15u;
+        const uint32_t i = tid + kT * u, s = i >> 4, c = i & 15u;
         const bool ok = slot_ok[s] != 0;
         vtile[s][c] = ok ? vw[u] : make_uint4(0, 0, 0, 0);
         if (s0 + s < count)
@@ -290,15 +298,16 @@ pack_kernel(PoolSource ps, MapSource ms, const uint64_t* __restrict__ positions,
                             ok ? kw[u] : make_uint4(0, 0, 0, 0));
     }
     __syncthreads();
-    // V[h][d][s]: 128 channel rows x 64 slots.  A thread gathers 8
+    // V[h][d][s]: 128 channel rows x kSlots.  A thread gathers 8
     // consecutive slots of one channel from the tile and stores them as one
-    // 16-byte word (8 threads cover a channel row's 128 B); rows whose start
+    // 16-byte word (kSlots / 8 threads cover a channel row); rows whose start
     // is not 16-byte aligned (count % 8 != 0) or that end inside the group
     // store element by element.
     const uint16_t* vt = reinterpret_cast<const uint16_t*>(&vtile[0][0]);
     const bool wide = (count & 7u) == 0 && (reinterpret_cast<uintptr_t>(v_out) & 15u) == 0;
-    for (uint32_t i = tid; i < 128 * 8; i += 256) {
-        const uint32_t d = i >> 3, sg = (i & 7u) * 8;
+    constexpr uint32_t kRuns = kSlots / 8;
+    for (uint32_t i = tid; i < 128 * kRuns; i += kT) {
+        const uint32_t d = i / kRuns, sg = (i % kRuns) * 8;
         uint32_t w[4];
 #pragma unroll
         for (uint32_t j = 0; j < 4; ++j)
@@ -317,8 +326,9 @@ pack_kernel(PoolSource ps, MapSource ms, const uint64_t* __restrict__ positions,
         // mask rows, 4 slots (16 B) per thread where the row allows
         const uint32_t qpad = (nq + 63) / 64 * 64;
         const bool wide_mask = (count & 3u) == 0 && (reinterpret_cast<uintptr_t>(mask) & 15u) == 0;
-        for (uint32_t i = tid; i < qpad * 16; i += 256) {
-            const uint32_t qi = i >> 4, sg = (i & 15u) * 4;
+        constexpr uint32_t kQuads = kSlots / 4;
+        for (uint32_t i = tid; i < qpad * kQuads; i += kT) {
+            const uint32_t qi = i / kQuads, sg = (i % kQuads) * 4;
             const uint64_t pos = qi < nq ? positions[qi] : 0;
             uint32_t m[4];  // 0 or -inf
 #pragma unroll
@@ -397,8 +407,9 @@ int hs_gqa_pack(const uint8_t* k_pool_dev, const uint8_t* v_pool_dev, size_t row
                       row_of_id_dev, max_id, ids_dev, lens_dev, static_cast<uint32_t>(ids_stride)};
     hs::MapSource ms{nullptr, nullptr, nullptr};
     hs::clear_status_if_captured(status_dev, 1, s);
-    hipLaunchKernelGGL(hs::pack_kernel<true>, dim3((count + 63) / 64, 32), dim3(256), 0, s, ps, ms,
-                       positions_dev, nq, count, k_dev, v_dev, mask_dev, status_dev,
+    const uint32_t slots = count <= hs::kShortSlots ? 32u : 64u;
+    hipLaunchKernelGGL((slots == 32 ? hs::pack_kernel<true, 32> : hs::pack_kernel<true, 64>),
+                       dim3((count + slots - 1) / slots, 32), dim3(slots * 4), 0, s, ps, ms, positions_dev, nq, count, k_dev, v_dev, mask_dev, status_dev,
                        hs::next_stamp());
     const hipError_t st = hipGetLastError();
     return st == hipSuccess ? HS_OK : hs::hip_fail(st, "pack launch");
@@ -417,8 +428,9 @@ int hs_gqa_gather_rows(const uint16_t* prefetched_dev, uint32_t prefetched_rows,
     hs::MapSource ms{prefetched_dev, misses_dev, map_dev, prefetched_rows, miss_rows};
     hipStream_t s = hs::as_stream(stream);
     hs::clear_status_if_captured(status_dev, 1, s);
-    hipLaunchKernelGGL(hs::pack_kernel<false>, dim3((count + 63) / 64, 32), dim3(256), 0, s, ps,
-                       ms, nullptr, 0u, count, k_dev, v_dev, nullptr, status_dev, hs::next_stamp());
+    const uint32_t slots = count <= hs::kShortSlots ? 32u : 64u;
+    hipLaunchKernelGGL((slots == 32 ? hs::pack_kernel<false, 32> : hs::pack_kernel<false, 64>),
+                       dim3((count + slots - 1) / slots, 32), dim3(slots * 4), 0, s, ps, ms, nullptr, 0u, count, k_dev, v_dev, nullptr, status_dev, hs::next_stamp());
     const hipError_t st = hipGetLastError();
     return st == hipSuccess ? HS_OK : hs::hip_fail(st, "gather launch");
 }

@@ -210,3 +210,31 @@ def test_union_bitmap_edges(hs, visible):
         out, out_n, status = hs.ops.physical_union(ids, lens, stride, visible)
         assert hs.ops.read_status(status)["code"] == hs.HS_ERR_DUPLICATE
         assert int(out_n.item()) == len(want)  # the refused id adds nothing
+
+
+@pytest.mark.parametrize("slots", [1, 31, 33, 4095, 4096, 4097, 4104])
+def test_slot_tile_edges(hs, port, slots):
+    # 32 slots per workgroup up to 4096 slots, 64 beyond: full and ragged last
+    # tiles, wide and element-wise stores, heads with fewer ids than slots
+    g = rng(30 + slots)
+    n = 4400
+    payload = g.integers(0, 256, size=n * 4096, dtype=np.uint8)
+    rows = g.permutation(n).astype(np.uint32)
+    selected = [g.choice(n, size=int(g.integers(max(1, slots - 40), slots + 1)), replace=False) for _ in range(32)]
+    queries = [n // 2, n - 1]
+    st, k, v, mask = gpu_pack(hs, selected, queries, rows, payload, slots)
+    rc, pk, pv, pmask = port.pack(selected, queries, rows, payload, slots)
+    assert st["code"] == 0 and rc == 0
+    assert np.array_equal(k, pk) and np.array_equal(v, pv)
+    assert np.array_equal(mask.view(np.uint32), pmask.view(np.uint32))
+    rec = payload.reshape(n, 4096)
+    row_map = np.full((32, slots), -1, dtype=np.int32)
+    for h in range(32):
+        s = selected[h].astype(np.int64)
+        row_map[h, : len(s)] = np.where(s < 3000, s, -2 - (s - 3000))
+    kd, vd, status = hs.ops.gather_rows(torch.from_numpy(rec[:3000].reshape(-1)).cuda(),
+                                        torch.from_numpy(rec[3000:].reshape(-1)).cuda(),
+                                        to_dev(row_map.reshape(-1)), slots)
+    gk, gv = port.gather_rows(rec[:3000].view(np.uint16), rec[3000:].view(np.uint16), row_map.reshape(-1), slots)
+    assert hs.ops.read_status(status)["code"] == 0
+    assert np.array_equal(from_dev(kd), gk) and np.array_equal(from_dev(vd), gv)
