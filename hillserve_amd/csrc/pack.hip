@@ -188,14 +188,16 @@ __device__ __forceinline__ const uint8_t* fallback_row(const PoolSource& ps, con
 // V cost more than the finer split gives (6560 slots: gather 43.5 -> 44.8, pack
 // 59.6 -> 62.2).
 // Bound by HBM: at 6560 slots the pack moves 269 MB (161 MB written), the
-// gather 215 MB (107 MB written).  The packed K, V and mask leave through
-// streaming stores: nothing here reads them back, and through the ordinary
-// path they push the pool rows, which the four query heads of a KV head
-// read again, out of the caches.  With both calls rotating over three sets
-// of buffers (before -> after): pack with its union, 6560 slots, 82.3 ->
-// 73.7 us; 3296 slots, 49.1 -> 37.6 us; gather of 6560 slots 45.6 -> 43.6 us,
-// of 1664 slots 11.6 -> 10.6 us.  (Streaming loads of the rows as well lose
-// that reuse: 76.3, 45.3, 44.5 and 13.4 us.)
+// gather 215 MB (107 MB written).  The packed V and mask leave through
+// streaming stores, K through the caches: with all three in the caches the
+// output pushes out the pool rows that the four query heads of a KV head read
+// again, with all three streamed a workspace reused from layer to layer no
+// longer stays in the MALL.  us, all cached / all streamed / as here: 6560
+// slots, three workspaces in turn: pack with its union 68.2 / 59.8 / 59.6,
+// gather 45.9 / 43.5 / 41.6; one workspace over 30 pools: pack 49.6 / 52.1 /
+// 48.3, gather 37.9 / 41.4 / 37.9; a 64-query pack of 1664 slots with its union
+// 17.9 / 17.6 / 16.7.  (Streaming loads of the rows lose their reuse: pack with
+// its union 76.3, gather 44.5.)
 constexpr uint32_t kShortSlots = 256 * 8 / 32 * 64;
 template <bool kPack, uint32_t kSlots>
 __global__ void __launch_bounds__(kSlots * 4)
@@ -294,8 +296,8 @@ pack_kernel(PoolSource ps, MapSource ms, const uint64_t* __restrict__ positions,
         const bool ok = slot_ok[s] != 0;
         vtile[s][c] = ok ? vw[u] : make_uint4(0, 0, 0, 0);
         if (s0 + s < count)
-            store_streaming(k_out + (static_cast<size_t>(s0 + s) * 32 + h) * 128 + 8 * c,
-                            ok ? kw[u] : make_uint4(0, 0, 0, 0));
+            reinterpret_cast<uint4*>(k_out + (static_cast<size_t>(s0 + s) * 32 + h) * 128)[c] =
+                ok ? kw[u] : make_uint4(0, 0, 0, 0);
     }
     __syncthreads();
     // V[h][d][s]: 128 channel rows x kSlots.  A thread gathers 8
