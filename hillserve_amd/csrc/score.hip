@@ -44,17 +44,18 @@ constexpr uint32_t kWavesPerBlock = 2;
 // read them again while the 256 MB MALL still holds them: they then stop
 // displacing the scores and dots that the next launches read, and a long
 // stream runs faster.  The dots' launch leaves the attention only V
-// rows to read, so its keys are done with: streamed from 56 MiB (28672
-// tokens), where the pools of a few layers no longer fit the MALL together.
-// One layer 46.0 -> 43.7 us at 32768 tokens, 73.5 -> 67.7 at 65536; below the
-// line it would lose what the MALL holds from the pass before (24576 tokens
-// 39.5 -> 41.3 us, 16384 33.2 -> 35.2).  A plain scoring launch is followed
+// rows to read, so its keys are done with: streamed from 72 MiB (36864
+// tokens).  One layer, ten pools in turn: 70.9 -> 68.7 us at 65536 tokens, 62.2
+// -> 61.7 at 40960, but 47.3 -> 47.5 at 32768 (44.8 -> 45.4 with 30 pools), where
+// only a few pools in turn gain (three: 46.0 -> 43.6), as their V rows then
+// stay in the MALL; below that it loses what the MALL holds from the pass
+// before (24576 tokens 39.5 -> 41.3).  A plain scoring launch is followed
 // by an attention that reads the selected K rows, so its line is 128 MiB,
 // more than the MALL keeps until then: 16 sequences of 8192 to 32768 tokens
-// 173.8 -> 155.8 us, a 65536-token cover 81.7 -> 77.4 us, while the pipelined
+// 173.8 -> 155.8 us, a 65536-token cover 67.9 -> 64.3 us, while the pipelined
 // 32768-token layers (64 MiB a launch) would lose 2.4 us each.
 constexpr uint64_t kStreamKeyBytes = uint64_t(128) << 20;
-constexpr uint64_t kStreamLogitKeyBytes = uint64_t(56) << 20;
+constexpr uint64_t kStreamLogitKeyBytes = uint64_t(72) << 20;
 
 template <bool kRows, bool kBatch, bool kStream>
 __global__ void __launch_bounds__(kWavesPerBlock * 64)

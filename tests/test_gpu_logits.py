@@ -84,9 +84,9 @@ def test_attention_from_dots(hs, port, n, frac, mapped):
     assert rel_err(got, via_k) <= 1e-3
 
 
-@pytest.mark.parametrize("n", [28671, 28672, 65536])
+@pytest.mark.parametrize("n", [36863, 36864, 65536])
 def test_streamed_keys(hs, n):
-    # keys are streamed from 28672 tokens in the dots' launch and from 65536
+    # keys are streamed from 36864 tokens in the dots' launch and from 65536
     # in plain scoring (single and batched): the same bits as calls below
     # those lines over parts of the keys
     keys = torch.empty(n * 1024, dtype=torch.float16, device="cuda")
