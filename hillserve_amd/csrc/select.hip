@@ -2253,7 +2253,13 @@ combine_count_kernel(const float* __restrict__ part, uint32_t chunks, float* __r
 
 }  // namespace
 
-size_t select_workspace_bytes(uint32_t heads, uint32_t n) { return plan_select(heads, n, n).total; }
+// Never less than a shorter sequence needs (past kHeadMaxN2 there are no order
+// keys, so the layout alone would shrink there): a workspace made for a
+// program's longest sequence serves every shorter one.
+size_t select_workspace_bytes(uint32_t heads, uint32_t n) {
+    const size_t own = plan_select(heads, n, n).total;
+    return n <= kHeadMaxN2 ? own : std::max(own, plan_select(heads, kHeadMaxN2, kHeadMaxN2).total);
+}
 
 namespace {
 

@@ -63,3 +63,23 @@ def test_c_program_links_and_calls(tmp_path):
     proc = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
     assert proc.returncode == 0, proc.stdout + proc.stderr
     assert '"failures":0' in proc.stdout, proc.stdout
+
+
+@pytest.mark.parametrize("size", ["hs_gqa_select_workspace_bytes", "hs_decode_layer_workspace_bytes",
+                                  "hs_gqa_attention_workspace_bytes"])
+def test_workspace_of_the_longest_sequence_serves_shorter(size):
+    # each layout change lies at a size of its own (8192, 16384, 32768 and
+    # 65536 tokens); no size up to it may need more than the size itself
+    import ctypes
+
+    import hillserve_amd
+    lib = ctypes.CDLL(str(Path(hillserve_amd.__file__).parent / "libhillserve_amd.so"))
+    f = getattr(lib, size)
+    f.restype = ctypes.c_size_t
+    lead = [32] if "select" in size else []
+    f.argtypes = [ctypes.c_uint32] * (len(lead) + 1)
+    most = 0
+    for n in range(1, 131073):
+        need = f(*lead, n)
+        assert need >= most, n
+        most = need
