@@ -54,6 +54,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "hs_device.hpp"
 #include "attention_combine.hpp"
@@ -1392,12 +1393,15 @@ static_assert(kSortRange % kHThreads == 0, "whole key bins per thread");
 // Capacities of one per-head workgroup.  kMaxK: composites in rank order;
 // kRound: composites compacted at a time (kW = 2 compacts each of a thread's
 // words in turn, since the LDS does not hold two lists of kHeadMaxK2); kStage:
-// ids staged in id order.
+// ids staged in id order (kW = 2: in 16 bits, so that half of 65536 fit the
+// LDS that two workgroups of a CU have each; 19660 of 65536 take 21.9 us, 27.9
+// past the stage).
 template <uint32_t kW>
 struct HeadCaps {
     static constexpr uint32_t kMaxK = kW == 1 ? kHeadMaxK : kHeadMaxK2;
     static constexpr uint32_t kRound = kHeadMaxK;
-    static constexpr uint32_t kStage = kW == 1 ? kHeadMaxK : 2 * kHeadMaxK;
+    static constexpr uint32_t kStage = kW == 1 ? kHeadMaxK : 4 * kHeadMaxK;
+    using StageId = std::conditional_t<kW == 1, uint32_t, uint16_t>;
 };
 
 // LDS of one per-head workgroup.
@@ -1413,7 +1417,7 @@ struct HeadSelectLds {
     // kW = 1: the radix sort's histograms, or a spare word per thread; kW = 2:
     // the spare words (the histograms take the compacted list's place)
     uint32_t whist[kRankOrder ? (kW == 1 ? kHWaves : kHThreads / 256) : 1][256];
-    uint32_t stage[kRankOrder ? 1 : Caps::kStage];  // id order: the ids before their store
+    typename Caps::StageId stage[kRankOrder ? 1 : Caps::kStage];  // id order: the ids before their store
 };
 static_assert(sizeof(HeadSelectLds<true, 2>) <= 160 * 1024, "one workgroup's LDS");
 
@@ -1666,18 +1670,31 @@ __device__ __forceinline__ void head_select(const SelectJobs& js, uint32_t h, ui
         if (k <= Caps::kStage) {
             // into LDS at their places, then out in row order: the stores of a
             // wave cover 256 consecutive bytes instead of 64 scattered places
-            uint32_t* stage = lds.stage;
+            auto* stage = lds.stage;
 #pragma unroll
             for (uint32_t w = 0; w < kW; ++w)
                 for (uint32_t sel = bits32[w]; sel != 0; sel &= sel - 1)
-                    stage[pos++] = begin + 32 * w + static_cast<uint32_t>(__ffs(sel)) - 1;
+                    stage[pos++] = static_cast<typename Caps::StageId>(
+                        begin + 32 * w + static_cast<uint32_t>(__ffs(sel)) - 1);
             __syncthreads();
             for (uint32_t r = tid; r < k; r += kHThreads) out[r] = stage[r];
         } else {
-#pragma unroll
-            for (uint32_t w = 0; w < kW; ++w)
-                for (uint32_t sel = bits32[w]; sel != 0; sel &= sel - 1)
-                    out[pos++] = begin + 32 * w + static_cast<uint32_t>(__ffs(sel)) - 1;
+            // a wave writes its words two at a time, lane = id, so a store's
+            // ids are consecutive: a thread's own ids stored one by one, or
+            // staged in parts (lanes 32 or 64 places apart: bank conflicts),
+            // take up to twice as long.  32 heads, every id: 65536 ids 51.7 ->
+            // 27.6 us (the slice launches: 25.9), 40000 40.1 -> 26.6 (27.0),
+            // 32768 30.9 -> 18.0
+            uint32_t at = __builtin_amdgcn_readfirstlane(pos);
+#pragma unroll 8
+            for (uint32_t t = 0; t < 64; t += 2 / kW) {
+                const uint32_t w0 = __builtin_amdgcn_readlane(bits32[0], t);
+                const uint32_t w1 = kW == 2 ? __builtin_amdgcn_readlane(bits32[kW - 1], t)
+                                            : __builtin_amdgcn_readlane(bits32[0], t + 1);
+                const uint64_t ids = (static_cast<uint64_t>(w1) << 32) | w0;
+                if ((ids >> lane) & 1u) out[at + lanes_below(ids)] = (tid - lane + t) * 32 * kW + lane;
+                at += static_cast<uint32_t>(__popcll(ids));
+            }
         }
     } else {
         // Rank order (k <= Caps::kMaxK here): a counting sort by key over the

@@ -448,6 +448,25 @@ def test_mixed_word_counts_in_a_batch(hs, port):
                 assert np.array_equal(from_dev(ids)[:, :k], np.sort(pids, axis=1) if id_order else pids)
 
 
+@pytest.mark.parametrize("n,k", [(20000, 8192), (20000, 8193), (20001, 20001), (32768, 32768), (32769, 16384),
+                                 (40001, 32768), (40001, 32769), (65535, 65535), (65536, 65536)])
+def test_id_order_around_the_stage(hs, port, n, k):
+    # the ids of one workgroup leave through its LDS stage (8192 of them up to
+    # 32768 tokens, 32768 beyond) or, past it, a wave's words at a time
+    g = rng(n + k)
+    heads = 3
+    s = f16_bits(g.standard_normal((heads, n)) * 2.0)
+    ratio = min(1.0, (k + 0.5) / n)
+    member = torch.zeros(heads * ((n + 31) // 32), dtype=torch.int32, device="cuda")
+    rc, kk, ids, _, tied = port.select(s, heads, n, n, 1000.0, ratio, True)
+    assert rc == 0 and kk == k
+    st, got, _, _ = gpu_select(hs, s, heads, n, n, 1000.0, ratio, fp32_counts=True, id_order=True, member=member)
+    assert st["code"] == 0 and st["k"] == k and st["boundary_tied_heads"] == tied
+    want = np.sort(ids, axis=1)
+    assert np.array_equal(got, want)
+    assert np.array_equal(from_dev(member).view(np.uint32).reshape(heads, -1), member_from_ids(want, n))
+
+
 @pytest.mark.parametrize("offset", range(8))
 def test_rows_off_sixteen_bytes(hs, port, offset):
     # score rows at every offset within 16 bytes (an odd stride, a base off by
