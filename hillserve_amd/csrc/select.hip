@@ -1108,6 +1108,64 @@ __device__ void sort_composites(uint32_t* A, uint32_t* B, uint32_t m, uint32_t (
     }
 }
 
+// The same stable sort in place, by one large workgroup: LSD radix, four bits
+// a pass.  Thread t holds kPer consecutive composites (kPer odd, so that their
+// reads do not conflict) and counts their digits in a column of its own, two
+// 16-bit counters to a word, so neither the counting nor a composite's rank
+// among its thread's needs a ballot; one scan over (digit, thread) then places
+// all.  (The composites are read again after it: in registers all the while
+// they would not leave enough to what the kernel holds.)  Its 13107 composites
+// of 65536 ids with 82 of a key take a selection of 32 heads 36.4 us in all,
+// with sort_composites 62.8, with the slice launches 60.0 (25.4 where no key
+// occurs more than 64 times); of one head 33.5, 59.9 and 34.6.
+// m <= kT kPer; passes: 4, or fewer where the keys agree in the digits above;
+// counts: 8 kT words; A: kT kPer words.
+template <uint32_t kT, uint32_t kPer>
+__device__ void sort_columns(uint32_t* A, uint32_t m, uint32_t passes, uint32_t* counts, uint32_t* tmp,
+                             uint32_t* low_total) {
+    static_assert(kPer % 2 == 1 && kPer < 16 && kT * kPer < 65536, "ranks of 4 bits, counts of 16");
+    const uint32_t tid = threadIdx.x;
+    for (uint32_t i = m + tid; i < kT * kPer; i += kT) A[i] = 0xffffffffu;  // past every composite
+    __syncthreads();
+#pragma unroll 1
+    for (uint32_t pass = 0; pass < passes; ++pass) {
+        const uint32_t shift = 16 + 4 * pass;
+#pragma unroll
+        for (uint32_t d = 0; d < 8; ++d) counts[d * kT + tid] = 0;
+        uint32_t ranks[2] = {0, 0};
+#pragma unroll
+        for (uint32_t u = 0; u < kPer; ++u) {
+            const uint32_t d = (A[tid * kPer + u] >> shift) & 15u;
+            const uint32_t old = atomicAdd(&counts[(d & 7u) * kT + tid], d & 8u ? 0x10000u : 1u);
+            ranks[u / 8] |= ((d & 8u ? old >> 16 : old) & 15u) << (4 * (u % 8));
+        }
+        __syncthreads();
+        // digits 0..7 in the low halves, 8..15 in the high ones
+        uint32_t sum = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i) sum += counts[8 * tid + i];
+        uint32_t run = block_exclusive_scan<kT>(sum, tmp);
+        if (tid == kT - 1) *low_total = (run + sum) & 0xffffu;
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i) {
+            const uint32_t c = counts[8 * tid + i];
+            counts[8 * tid + i] = run;
+            run += c;
+        }
+        uint32_t x[kPer];
+#pragma unroll
+        for (uint32_t u = 0; u < kPer; ++u) x[u] = A[tid * kPer + u];
+        __syncthreads();
+        const uint32_t low = *low_total;
+#pragma unroll
+        for (uint32_t u = 0; u < kPer; ++u) {
+            const uint32_t d = (x[u] >> shift) & 15u, at = counts[(d & 7u) * kT + tid];
+            A[(d & 8u ? (at >> 16) + low : at & 0xffffu) + ((ranks[u / 8] >> (4 * (u % 8))) & 15u)] = x[u];
+        }
+        __syncthreads();
+    }
+}
+
 // Counting sort of m composites ((0xffff - key) << 16 | id in slice) in A,
 // using B, when the keys span at most kSortRange values from kmin and no key
 // occurs more than kGroupCap times: key histogram, exclusive suffix scan
@@ -1415,7 +1473,7 @@ struct HeadSelectLds {
     uint32_t sort_lds[kRankOrder ? Caps::kMaxK + 8 + Caps::kRound : 1];
     alignas(16) uint32_t tables[kRankOrder ? 2 * kSortRange : 1];
     // kW = 1: the radix sort's histograms, or a spare word per thread; kW = 2:
-    // the spare words (the histograms take the compacted list's place)
+    // the spare words
     uint32_t whist[kRankOrder ? (kW == 1 ? kHWaves : kHThreads / 256) : 1][256];
     typename Caps::StageId stage[kRankOrder ? 1 : Caps::kStage];  // id order: the ids before their store
 };
@@ -1796,22 +1854,51 @@ __device__ __forceinline__ void head_select(const SelectJobs& js, uint32_t h, ui
             // a long run of equal keys or a key range past the table: stable
             // radix sort of the composites written in id order
             uint32_t* A = sort_lds;
-#pragma unroll
-            for (uint32_t w = 0; w < kW; ++w)
+            if constexpr (kW == 1) {
 #pragma unroll
                 for (uint32_t j = 0; j < 32; ++j) {
-                    if ((bits32[w] >> j) & 1u) {
-                        const uint32_t key = half_at(keys[w], j);
-                        A[pos++] = ((0xffffu - key) << 16) | (begin + 32 * w + j);
+                    if ((bits32[0] >> j) & 1u) {
+                        const uint32_t key = half_at(keys[0], j);
+                        A[pos++] = ((0xffffu - key) << 16) | (begin + j);
                     }
                 }
-            __syncthreads();
-            if constexpr (kW == 1) {
+                __syncthreads();
                 sort_composites<kHThreads>(A, A + kHeadMaxK, m, whist, tmp);
-            } else {  // the tables and the compacted list are free here
-                static_assert(2 * kSortRange >= Caps::kMaxK && Caps::kRound >= kHWaves * 256, "room for the sort");
-                sort_composites<kHThreads>(A, tables, m,
-                                           reinterpret_cast<uint32_t(*)[256]>(sort_lds + Caps::kMaxK + 8), tmp);
+            } else {
+                // the ids, then their keys from the workspace again (held in
+                // registers up to here they left none for the sort)
+#pragma unroll
+                for (uint32_t w = 0; w < kW; ++w)
+                    for (uint32_t sel = bits32[w]; sel != 0; sel &= sel - 1)
+                        A[pos++] = begin + 32 * w + static_cast<uint32_t>(__ffs(sel)) - 1;
+                __syncthreads();
+                for (uint32_t i = tid; i < m; i += kHThreads) {
+                    const uint32_t id = A[i];
+                    const uint32_t key = krow[key_chunk(id / 32, (id / 8) & 3u, a.key_stride) + (id & 7u)];
+                    A[i] = ((0xffffu - key) << 16) | id;
+                }
+                __syncthreads();
+                // all selected keys agree in the digits that no key of the head
+                // exceeds K*'s in
+                const uint32_t bucket = kstar >> 8;
+                bool past_bucket = false, past_digit = false;
+#pragma unroll
+                for (uint32_t u = 0; u < 4; ++u) {
+                    const uint32_t b = lane + 64 * u;
+                    const bool some = hist[0][b] != 0;
+                    past_bucket |= some && b > bucket;
+                    past_digit |= some && b > (bucket | 15u);
+                }
+                const uint32_t passes = __ballot(past_digit) ? 4u : __ballot(past_bucket) ? 3u : 2u;
+                // (the tables are free here)
+                constexpr uint32_t kPerThread = Caps::kMaxK / kHThreads;
+                static_assert(kPerThread * kHThreads == Caps::kMaxK && kSortRange == 8 * kHThreads, "room for the sort");
+                if (m <= kHThreads)
+                    sort_columns<kHThreads, 1>(A, m, passes, tables, tmp, &sh[kRounds]);
+                else if (m <= 5 * kHThreads)
+                    sort_columns<kHThreads, 5>(A, m, passes, tables, tmp, &sh[kRounds]);
+                else
+                    sort_columns<kHThreads, kPerThread>(A, m, passes, tables, tmp, &sh[kRounds]);
             }
             for (uint32_t r = tid; r < m; r += kHThreads) out[r] = A[r] & 0xffffu;
         }

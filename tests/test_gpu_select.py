@@ -448,6 +448,33 @@ def test_mixed_word_counts_in_a_batch(hs, port):
                 assert np.array_equal(from_dev(ids)[:, :k], np.sort(pids, axis=1) if id_order else pids)
 
 
+@pytest.mark.parametrize("span", ["bucket", "digit", "sign"])
+@pytest.mark.parametrize("k", [1, 1023, 1024, 1025, 5120, 5121, 13107, 13312])
+def test_long_runs_past_32768(hs, port, span, k):
+    # more than 64 equal keys past 32768 ids: the radix sort, with one, five or
+    # thirteen composites per thread, and two, three or four digits by how far
+    # the selected keys reach (one high byte, one top digit, both signs)
+    g = rng(700 + k + len(span))
+    heads, n = 2, 65536
+    # (k at the cap; the lowest scores of every head are filling)
+    s = np.full((heads, n), hb(-60000), dtype=np.uint16)
+    few = {"bucket": np.arange(0x4a00, 0x4a28), "digit": np.arange(0x4410, 0x47f0, 61),
+           "sign": f16_bits(np.linspace(-3.0, 3.0, 41))}[span].astype(np.uint16)
+    for h in range(heads):
+        at = g.choice(n, size=k, replace=False)
+        s[h, at] = g.choice(few, size=k)
+        s[h, at[: min(k, 80)]] = few[-1]
+    alpha, ratio = 65504.0, (k + 0.5) / n
+    rc, kk, ids, _, _ = port.select(s, heads, n, n, alpha, ratio, True)
+    assert rc == 0 and kk == k
+    keys = order_keys(s[np.arange(heads)[:, None], ids])
+    if k > 1000:
+        reach = {"bucket": (0, 0), "digit": (1, 0), "sign": (1, 1)}[span]
+        assert (len(np.unique(keys >> 8)) > 1, len(np.unique(keys >> 12)) > 1) == reach
+        assert max(np.unique(row, return_counts=True)[1].max() for row in keys) > 64
+    check_against_port(hs, port, s, heads, n, n, alpha, ratio, True)
+
+
 @pytest.mark.parametrize("n,k", [(20000, 8192), (20000, 8193), (20001, 20001), (32768, 32768), (32769, 16384),
                                  (40001, 32768), (40001, 32769), (65535, 65535), (65536, 65536)])
 def test_id_order_around_the_stage(hs, port, n, k):
