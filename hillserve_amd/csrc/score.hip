@@ -82,13 +82,20 @@ score_logits_kernel(const ScoreJobs jobs, const int32_t* __restrict__ rows, uint
 }
 
 // Up to kShortIds (token tile, KV head) pairs, four per CU: a wave of its own
-// workgroup for each, spread over all CUs, both halves of its tile in flight
-// at once (in two-wave workgroups half the CUs would hold two waves, and
-// the second half waits for the first).  One layer of 1024 tokens 19.6 -> 19.1
-// us, of 7919 in 4096 B records 27.4 -> 26.9, of 8192 26.4 -> 24.8; score, cover
-// and union of 1024 24.4 -> 24.1.  From 12288 tokens on the waves fill the CUs
-// and it is slower (30.8 -> 31.5 us a layer).
+// workgroup for each, spread over all CUs (in two-wave workgroups half the CUs
+// would hold two waves): 16 pools scored in turn 104.1 -> 95.4 us at 8192
+// tokens, 69.4 -> 66.4 at 1024, a layer of 8192 29.2 -> 24.1 with the launch
+// after it.  From 12288 tokens on the waves fill the CUs and it is slower
+// (30.8 -> 31.5 us a layer).
 constexpr uint32_t kShortIds = 1024;
+// Both halves of a wave's tile are in flight at once (the second otherwise
+// waits for the first) in the dots' launch, and in plain scoring up to
+// kOneTileIds, a wave on each CU.  16 pools in turn, both at once / one after
+// the other: plain 64.7 / 66.4 us at 1024 tokens, 66.9 / 67.6 at 2048, but
+// 73.2 / 70.9 at 3072, 77.5 / 73.4 at 4096 (74.6 with two-wave workgroups)
+// and 104.9 / 95.4 at 8192; layers 308.0 / 311.5 at 1024, 355.9 / 354.1 at
+// 4096, 399.8 / 402.0 at 5120, 436.3 / 430.3 at 8192.
+constexpr uint32_t kOneTileIds = 256;
 static_assert(kShortIds >= kShortTokens / kTileTokens * 8, "the launches that clear the exchange words");
 
 // By one wave of the launch before launch_layer_select.
@@ -100,11 +107,11 @@ __device__ __forceinline__ void clear_exchange(const SelectExchange& clear) {
     if (lane == 0) *clear.tied_heads = 0;
 }
 
-template <bool kRows, bool kBatch>
+template <bool kRows, bool kBatch, bool kOneTile>
 __global__ void __launch_bounds__(64)
 score_short_kernel(const ScoreJobs jobs, const int32_t* __restrict__ rows, uint32_t pool_rows) {
     __shared__ uint4 lds[kHalfTileChunks];
-    score_waves<kRows, kBatch, false, false, true>(jobs, rows, pool_rows, blockIdx.x, gridDim.x, lds);
+    score_waves<kRows, kBatch, false, false, kOneTile>(jobs, rows, pool_rows, blockIdx.x, gridDim.x, lds);
 }
 template <bool kRows>
 __global__ void __launch_bounds__(64)
@@ -160,7 +167,9 @@ int launch_score(const uint16_t* q, const uint16_t* keys, size_t stride_words,
             hipLaunchKernelGGL((rows ? score_logits_short_kernel<true> : score_logits_short_kernel<false>),
                                short_grid, wave, 0, stream, jobs, rows, rows ? pool_rows : 0u, lo, clear);
         else
-            hipLaunchKernelGGL((rows ? score_short_kernel<true, false> : score_short_kernel<false, false>),
+            hipLaunchKernelGGL((jobs.total_ids <= kOneTileIds
+                                    ? (rows ? score_short_kernel<true, false, true> : score_short_kernel<false, false, true>)
+                                    : (rows ? score_short_kernel<true, false, false> : score_short_kernel<false, false, false>)),
                                short_grid, wave, 0, stream, jobs, rows, rows ? pool_rows : 0u);
         const hipError_t status = hipGetLastError();
         return status == hipSuccess ? HS_OK : hip_fail(status, "score launch");
@@ -210,8 +219,9 @@ int launch_score_batched(const hs_score_job_t* jobs, uint32_t count, hipStream_t
     uint64_t key_bytes = 0;
     for (uint32_t i = 0; i < count; ++i) key_bytes += uint64_t(jobs[i].tokens) * 2048;
     if (table.total_ids <= kShortIds) {
-        hipLaunchKernelGGL((score_short_kernel<false, true>), dim3(table.total_ids), dim3(64), 0, stream,
-                           table, nullptr, 0u);
+        hipLaunchKernelGGL((table.total_ids <= kOneTileIds ? score_short_kernel<false, true, true>
+                                                           : score_short_kernel<false, true, false>),
+                           dim3(table.total_ids), dim3(64), 0, stream, table, nullptr, 0u);
     } else {
         const auto kernel = key_bytes >= kStreamKeyBytes ? score_kernel<false, true, true>
                                                          : score_kernel<false, true, false>;

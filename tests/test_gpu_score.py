@@ -121,11 +121,12 @@ def test_head0_partial_maxima(hs, port):
     assert np.array_equal(from_dev(partial), np.array(expected, dtype=np.uint32))
 
 
-@pytest.mark.parametrize("n", [1, 63, 64, 65, 8128, 8192, 8193])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 2047, 2048, 2049, 8128, 8192, 8193])
 def test_one_wave_per_tile(hs, port, n):
-    # up to 8192 tokens every (token tile, KV head) pair has a wave of its own
-    # that requests both halves of its tile at once: single and batched,
-    # plain and with the attention's dots, with a row map
+    # up to 8192 tokens every (token tile, KV head) pair has a wave of its own,
+    # which up to 2048 (with the dots up to 8192) requests both halves of its
+    # tile at once: single and batched, plain and with the attention's dots,
+    # with a row map
     g = rng(30 + n)
     q, k = mixed_finite(g, (32, 128)), mixed_finite(g, (n, 8, 128))
     want = port.score(q, k.reshape(-1), n, 1024)
