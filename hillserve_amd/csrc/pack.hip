@@ -183,10 +183,16 @@ __device__ __forceinline__ const uint8_t* fallback_row(const PoolSource& ps, con
 
 // Grid (ceil(count/kSlots), 32 heads), 4 threads per slot.  kPack selects the
 // source.  64 slots at a time; 32 up to kShortSlots, where 64 would leave the
-// chip's 8 workgroups per CU unfilled (gather of 1664 slots 10.6 -> 9.4 us, pack
-// of 3296 slots with its union 28.8 -> 28.0) and above which the shorter runs of
-// V cost more than the finer split gives (6560 slots: gather 43.5 -> 44.8, pack
-// 59.6 -> 62.2).
+// chip's 8 workgroups per CU unfilled (one workspace: gather of 1664 slots 9.6
+// -> 8.3 us, of 3296 18.1 -> 17.1, pack of 3296 22.5 -> 21.7) and above which
+// the shorter runs of V cost more than the finer split gives (6560 slots:
+// gather 43.5 -> 44.8, pack 59.6 -> 62.2).  Where the V rows are whole 128-byte
+// lines apart (slots a multiple of 64) 64 slots write whole lines and 32 half
+// ones, which costs more than the split gives from kLineSlots on once the
+// output is not in a cache.  Eight workspaces in turn, 32 / 64 slots: gather of
+// 3072 190.6 / 169.6 us, 3584 212.1 / 192.6, 4096 239.6 / 215.4, pack 216.8 /
+// 197.3, 248.1 / 227.9, 281.0 / 259.9, but 1664 103.6 / 108.1 and 3296 195.9 /
+// 195.1, 227.6 / 238.9; one workspace 16.0 / 16.4, 19.3 / 18.9, 21.5 / 21.8.
 // Bound by HBM: at 6560 slots the pack moves 269 MB (161 MB written), the
 // gather 215 MB (107 MB written).  The packed V and mask leave through
 // streaming stores, K through the caches: with all three in the caches the
@@ -198,7 +204,10 @@ __device__ __forceinline__ const uint8_t* fallback_row(const PoolSource& ps, con
 // 48.3, gather 37.9 / 41.4 / 37.9; a 64-query pack of 1664 slots with its union
 // 17.9 / 17.6 / 16.7.  (Streaming loads of the rows lose their reuse: pack with
 // its union 76.3, gather 44.5.)
-constexpr uint32_t kShortSlots = 256 * 8 / 32 * 64;
+constexpr uint32_t kShortSlots = 256 * 8 / 32 * 64, kLineSlots = 2560;
+inline uint32_t pack_slots(uint32_t count) {
+    return count <= kShortSlots && (count < kLineSlots || count % 64 != 0) ? 32u : 64u;
+}
 template <bool kPack, uint32_t kSlots>
 __global__ void __launch_bounds__(kSlots * 4)
 pack_kernel(PoolSource ps, MapSource ms, const uint64_t* __restrict__ positions, uint32_t nq,
@@ -409,10 +418,10 @@ int hs_gqa_pack(const uint8_t* k_pool_dev, const uint8_t* v_pool_dev, size_t row
                       row_of_id_dev, max_id, ids_dev, lens_dev, static_cast<uint32_t>(ids_stride)};
     hs::MapSource ms{nullptr, nullptr, nullptr};
     hs::clear_status_if_captured(status_dev, 1, s);
-    const uint32_t slots = count <= hs::kShortSlots ? 32u : 64u;
+    const uint32_t slots = hs::pack_slots(count);
     hipLaunchKernelGGL((slots == 32 ? hs::pack_kernel<true, 32> : hs::pack_kernel<true, 64>),
-                       dim3((count + slots - 1) / slots, 32), dim3(slots * 4), 0, s, ps, ms, positions_dev, nq, count, k_dev, v_dev, mask_dev, status_dev,
-                       hs::next_stamp());
+                       dim3((count + slots - 1) / slots, 32), dim3(slots * 4), 0, s, ps, ms,
+                       positions_dev, nq, count, k_dev, v_dev, mask_dev, status_dev, hs::next_stamp());
     const hipError_t st = hipGetLastError();
     return st == hipSuccess ? HS_OK : hs::hip_fail(st, "pack launch");
 }
@@ -430,9 +439,10 @@ int hs_gqa_gather_rows(const uint16_t* prefetched_dev, uint32_t prefetched_rows,
     hs::MapSource ms{prefetched_dev, misses_dev, map_dev, prefetched_rows, miss_rows};
     hipStream_t s = hs::as_stream(stream);
     hs::clear_status_if_captured(status_dev, 1, s);
-    const uint32_t slots = count <= hs::kShortSlots ? 32u : 64u;
+    const uint32_t slots = hs::pack_slots(count);
     hipLaunchKernelGGL((slots == 32 ? hs::pack_kernel<false, 32> : hs::pack_kernel<false, 64>),
-                       dim3((count + slots - 1) / slots, 32), dim3(slots * 4), 0, s, ps, ms, nullptr, 0u, count, k_dev, v_dev, nullptr, status_dev, hs::next_stamp());
+                       dim3((count + slots - 1) / slots, 32), dim3(slots * 4), 0, s, ps, ms, nullptr,
+                       0u, count, k_dev, v_dev, nullptr, status_dev, hs::next_stamp());
     const hipError_t st = hipGetLastError();
     return st == hipSuccess ? HS_OK : hs::hip_fail(st, "gather launch");
 }

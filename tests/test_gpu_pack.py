@@ -212,10 +212,11 @@ def test_union_bitmap_edges(hs, visible):
         assert int(out_n.item()) == len(want)  # the refused id adds nothing
 
 
-@pytest.mark.parametrize("slots", [1, 31, 33, 4095, 4096, 4097, 4104])
+@pytest.mark.parametrize("slots", [1, 31, 33, 2496, 2559, 2560, 2561, 2592, 4064, 4095, 4096, 4097, 4104])
 def test_slot_tile_edges(hs, port, slots):
-    # 32 slots per workgroup up to 4096 slots, 64 beyond: full and ragged last
-    # tiles, wide and element-wise stores, heads with fewer ids than slots
+    # 32 slots per workgroup up to 4096 slots, except for multiples of 64 from
+    # 2560, and 64 for those and beyond: full and ragged last tiles, wide and
+    # element-wise stores, heads with fewer ids than slots
     g = rng(30 + slots)
     n = 4400
     payload = g.integers(0, 256, size=n * 4096, dtype=np.uint8)
