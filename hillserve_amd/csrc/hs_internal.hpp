@@ -70,7 +70,7 @@ int launch_select(const uint16_t* scores, uint32_t heads, size_t stride, uint32_
 // The selection of hs_decode_layer (32 heads, stride n, id order) after a scoring
 // launch that cleared select_exchange's words.  wait_ticks (of 10 ns): how long
 // a workgroup of the short-sequence launch waits for the other heads' counts
-// before it counts the missing heads itself.
+// before it counts the missing heads itself (0: it counts them all).
 constexpr uint32_t kExchangeTicks = 5000;
 int launch_layer_select(const uint16_t* scores, uint32_t n, float alpha, float ratio, uint32_t flags,
                         const uint32_t* head0_partial, uint32_t* ids, size_t ids_stride,

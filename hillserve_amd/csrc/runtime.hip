@@ -166,7 +166,8 @@ int decode_layer(const uint16_t* q16_dev, const float* q32_dev, const uint8_t* k
                  const uint8_t* v_pool_dev, size_t row_bytes, const int32_t* row_of_id_dev,
                  uint32_t pool_rows, uint32_t n, float alpha, float ratio, uint32_t flags,
                  uint16_t* scores_dev, uint32_t* ids_dev, size_t ids_stride, uint32_t* counts_dev,
-                 float* out_dev, hs_status_t* status_dev, void* workspace_dev, hipStream_t s) {
+                 float* out_dev, hs_status_t* status_dev, void* workspace_dev, hipStream_t s,
+                 uint32_t wait_ticks = kExchangeTicks) {
     if (!q16_dev || !q32_dev || !k_pool_dev || !v_pool_dev || !scores_dev || !ids_dev ||
         !out_dev || !status_dev || !workspace_dev)
         return reject("decode layer: null pointer");
@@ -198,7 +199,7 @@ int decode_layer(const uint16_t* q16_dev, const float* q32_dev, const uint8_t* k
                       select_exchange(n, ratio, sel_flags, status_dev, ws + p.off_select));
     if (rc != HS_OK) return rc;
     rc = launch_layer_select(scores_dev, n, alpha, ratio, sel_flags, partial, ids_dev, ids_stride,
-                             counts_dev, member, status_dev, ws + p.off_select, s);
+                             counts_dev, member, status_dev, ws + p.off_select, s, wait_ticks);
     if (rc != HS_OK) return rc;
     return launch_attention_logits(logits, n, v_pool_dev, row_bytes, row_of_id_dev, pool_rows, member,
                                    n, out_dev, ws + p.off_attn, s);
@@ -269,6 +270,22 @@ int hs_selftest_key_table(uint16_t* keys_dev, void* stream) {
                        reinterpret_cast<uint32_t*>(keys_dev));
     const hipError_t st = hipGetLastError();
     return st == hipSuccess ? HS_OK : hs::hip_fail(st, "selftest launch");
+}
+
+int hs_selftest_decode_layer(const uint16_t* q16_dev, const float* q32_dev, const uint8_t* k_pool_dev,
+                             const uint8_t* v_pool_dev, size_t row_bytes,
+                             const int32_t* row_of_id_dev, uint32_t pool_rows, uint32_t n,
+                             float alpha, float ratio, uint32_t flags, uint16_t* scores_dev,
+                             uint32_t* ids_dev, size_t ids_stride, uint32_t* counts_dev,
+                             float* out_dev, hs_status_t* status_dev, void* workspace_dev,
+                             uint32_t wait_ticks, void* stream) {
+    hs::clear_error();
+    if (!workspace_dev) return hs::reject("decode layer: null pointer");
+    if (wait_ticks > hs::kExchangeTicks) return hs::reject("selftest: wait limit too long");
+    return hs::decode_layer(q16_dev, q32_dev, k_pool_dev, v_pool_dev, row_bytes, row_of_id_dev,
+                            pool_rows, n, alpha, ratio, flags, scores_dev, ids_dev, ids_stride,
+                            counts_dev, out_dev, status_dev, workspace_dev, hs::as_stream(stream),
+                            wait_ticks);
 }
 
 int hs_fill_gaussian_f16(uint16_t* dst_dev, size_t count, uint64_t seed, float scale,

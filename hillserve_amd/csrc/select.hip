@@ -1996,7 +1996,12 @@ __global__ void __launch_bounds__(kT) small_select_kernel(const SelectJobs js, u
         const uint64_t start = realtime_ticks();
         uint32_t word[kMaxHeads / 64];
         uint64_t left[kMaxHeads / 64];
-        bool wait = true;
+#pragma unroll
+        for (uint32_t u = 0; u < kMaxHeads / 64; ++u) {
+            word[u] = 0;
+            left[u] = __ballot(lane + 64 * u < a.heads);
+        }
+        bool wait = wait_ticks != 0;  // (0: not one word is read, every head is missing)
         while (wait) {
             wait = false;
 #pragma unroll

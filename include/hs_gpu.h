@@ -462,6 +462,18 @@ int hs_selftest_scale_table(uint16_t *table_dev, void *stream);
  * keys_dev [2][65536] (4-byte aligned), row 0 of the scaled values, row 1 of
  * the raw ones (entries of inf / NaN inputs are not meaningful) */
 int hs_selftest_key_table(uint16_t *keys_dev, void *stream);
+/* hs_decode_layer whose single launch of count and selection (up to 8192
+ * tokens) waits at most wait_ticks of 10 ns (0..5000, the limit of
+ * hs_decode_layer) for the other heads' counts before each head's workgroup
+ * counts the missing heads itself; 0: it counts all of them.  The results are
+ * the same. */
+int hs_selftest_decode_layer(const uint16_t *q16_dev, const float *q32_dev,
+                             const uint8_t *k_pool_dev, const uint8_t *v_pool_dev,
+                             size_t row_bytes, const int32_t *row_of_id_dev, uint32_t pool_rows,
+                             uint32_t n, float alpha, float ratio, uint32_t flags,
+                             uint16_t *scores_dev, uint32_t *ids_dev, size_t ids_stride,
+                             uint32_t *counts_dev, float *out_dev, hs_status_t *status_dev,
+                             void *workspace_dev, uint32_t wait_ticks, void *stream);
 
 /* ---- synthetic inputs (bench and tests; generated on device) -------------
  * Deterministic counter-based generator: value i of stream `seed` is a

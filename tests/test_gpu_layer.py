@@ -143,42 +143,79 @@ def test_short_layer_errors(hs, port):
         assert st["code"] == code and (st["k"] == 600) == (code == 0)
 
 
+@pytest.mark.parametrize("wait", [0, 1, 5000])
 @pytest.mark.parametrize("n", [1500, 3001, 8192])
-def test_short_layer_counts_missing_heads(hs, port, n):
-    # a workgroup that stops waiting for the other heads' counts at once
-    # counts them itself: the same selection, errors included
+def test_short_layer_counts_missing_heads(hs, port, n, wait):
+    # a workgroup that reads no other head's count (wait 0), or only those
+    # published by its first look, counts the rest itself: the same layer,
+    # errors included, on a workspace whose words all look published
     import ctypes
-    import subprocess
-    names = subprocess.run(["nm", "-D", "--defined-only", str(hs.LIB_PATH)], capture_output=True, text=True,
-                           check=True).stdout.split()
-    fn = getattr(hs.lib(), next(x for x in names if "launch_layer_select" in x))
-    P, U = ctypes.c_void_p, ctypes.c_uint32
-    fn.restype = ctypes.c_int
-    fn.argtypes = [P, U, ctypes.c_float, ctypes.c_float, U, P, P, ctypes.c_size_t, P, P, P, P, P, U]
-    flags = hs.HS_SELECT_SCALE_RAW | hs.HS_SELECT_REQUIRE_K | hs.HS_SELECT_ID_ORDER
     g = rng(n)
-    for bad in (None, 0, 9):
-        raw = f16_bits(g.standard_normal((32, n)) * 20.0)
+    k, v = rope_keys(n, n), f16_bits(g.standard_normal((n, 8, 128)))
+    q16 = f16_bits(g.standard_normal((32, 128)))
+    q32 = g.standard_normal((32, 128)).astype(np.float32)
+    kmax = int(np.floor(n * np.float64(np.float32(0.2))))
+    dev = lambda shape, dt=torch.int32: torch.full(shape, -1, dtype=dt, device="cuda")
+    P = lambda t: ctypes.c_void_p(t.data_ptr())
+    ws = torch.full((hs.ops.decode_layer_workspace_bytes(n),), 0xFF, dtype=torch.uint8, device="cuda")
+    for bad in (None, 0, 5):  # KV heads with a nonfinite key
+        kk = k.copy()
         if bad is not None:
-            raw[bad, n // 2] = 0x7E00
-        key = lambda b: np.where(b > 0x8000, b ^ 0xFFFF, (b & 0x7FFF) | 0x8000).astype(np.uint32)
-        keys = np.where((raw[0] & 0x7FFF) > 0x7C00, 0, key(raw[0]))
-        part = np.maximum.reduceat(keys, np.arange(0, n, 64)).astype(np.uint32)
-        kmax = int(np.floor(n * np.float64(np.float32(0.2))))
-        ids = torch.zeros((32, kmax), dtype=torch.int32, device="cuda")
-        counts = torch.zeros(32, dtype=torch.int32, device="cuda")
-        member = torch.zeros((32, (n + 31) // 32), dtype=torch.int32, device="cuda")
-        status = hs.ops.new_status()
-        ws = torch.zeros(hs.ops.select_workspace_bytes(32, n), dtype=torch.uint8, device="cuda")
-        raw_d, part_d = to_dev(raw), to_dev(part)
-        p = lambda t: t.data_ptr()
-        assert fn(p(raw_d), n, 3.0, 0.2, flags, p(part_d), p(ids), kmax, p(counts), p(member), p(status), p(ws),
-                  torch.cuda.current_stream().cuda_stream, 0) == 0
+            kk[n // 2, bad] = 0x7C00  # inf: its products are inf or NaN
+        pool = pool_rows(kk, v)
+        pd, q16d, q32d = to_dev(pool.reshape(-1)), to_dev(q16), torch.from_numpy(q32).cuda()
+        scores, ids, counts = dev((32, n), torch.float16), dev((32, kmax)), dev((32,))
+        out, status = dev((32, 128), torch.float32), dev((4,))
+        ws.fill_(0xFF)
+        hs.check(hs.lib().hs_selftest_decode_layer(
+            P(q16d), P(q32d), P(pd), ctypes.c_void_p(pd.data_ptr() + 2048), 4096, None, n, n, 4.0, 0.2, 0,
+            P(scores), P(ids), kmax, P(counts), P(out), P(status), P(ws), wait,
+            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
         st = hs.ops.read_status(status)
         if bad is not None:
-            assert st["code"] == hs.HS_ERR_NONFINITE and not from_dev(member).any()
+            assert st["code"] == hs.HS_ERR_NONFINITE
             continue
-        rc, k, pids, pcounts, tied = port.select(port.scale(raw), 32, n, n, 3.0, 0.2)
-        assert rc == st["code"] == 0 and st["k"] == k and st["boundary_tied_heads"] == tied
+        raw = port.score(q16, pool.reshape(-1), n, 2048)
+        rc, k_want, pids, pcounts, tied = port.select(port.scale(raw), 32, n, n, 4.0, 0.2)
+        assert np.array_equal(from_dev(scores), raw)
+        assert rc == st["code"] == 0 and st["k"] == k_want > 0 and st["boundary_tied_heads"] == tied
         assert np.array_equal(from_dev(counts), pcounts)
-        assert np.array_equal(from_dev(ids)[:, :k], np.sort(pids, axis=1))
+        assert np.array_equal(from_dev(ids)[:, :k_want], np.sort(pids, axis=1))
+        ref = port.attention(q32, pool.view(np.uint8).reshape(-1), [list(r) for r in pids])
+        assert rel_err(out.cpu().numpy().astype(np.float64), ref) <= 2e-3
+
+
+def test_selftest_layer_refuses_long_waits(hs):
+    import ctypes
+    assert hs.lib().hs_selftest_decode_layer(*[None] * 4, 4096, None, 1, 1, 1.0, 0.2, 0, None, None, 1, None, None,
+                                             None, ctypes.c_void_p(256), 5001, None) == hs.HS_ERR_ARGUMENT
+    assert "wait limit" in hs.last_error()
+
+
+@pytest.mark.parametrize("n", [3001, 8192, 12001, 16384, 40001, 65536])
+@pytest.mark.parametrize("row_bytes", [2048, 4096])
+def test_row_mapped_layer_equals_plain(hs, n, row_bytes):
+    # hs_decode_layer over a shuffled pool behind a row map, in every regime
+    # of its launches (one launch of count and selection, chunks of 32, 64 and
+    # 128 ids, streamed keys, two words per thread), as K and V arrays and as
+    # KV records: every output equals the plain layer's bit for bit
+    keys = torch.empty(n * 1024, dtype=torch.float16, device="cuda")
+    values, q16 = torch.empty_like(keys), torch.empty(4096, dtype=torch.float16, device="cuda")
+    hs.ops.fill_rope_keys(keys, n, 1024, 8, seed=n)
+    hs.ops.fill_gaussian(values, seed=n + 1)
+    hs.ops.fill_gaussian(q16, seed=n + 2)
+    q32 = torch.randn((32, 128), generator=torch.Generator(device="cuda").manual_seed(n), device="cuda")
+    k, v = keys.view(n, 1024), values.view(n, 1024)
+    want = hs.ops.decode_layer(q16, q32, k, n, 5.0, 0.2, v_pool=v, row_bytes=2048)
+    rows = n + 37  # rows of no token among them
+    g = rng(n)
+    place = torch.from_numpy(g.permutation(rows)[:n].astype(np.int64)).cuda()
+    mk, mv = (torch.full((rows, 1024), float("nan"), dtype=torch.float16, device="cuda") for _ in range(2))
+    mk[place], mv[place] = k, v
+    pool = dict(pool=mk, v_pool=mv) if row_bytes == 2048 else dict(pool=torch.cat([mk, mv], dim=1).contiguous())
+    got = hs.ops.decode_layer(q16, q32, pool.pop("pool"), n, 5.0, 0.2, rows=place.int(), row_bytes=row_bytes, **pool)
+    st = hs.ops.read_status(want[4])
+    assert hs.ops.read_status(got[4]) == st and st["code"] == 0 and st["k"] > 0
+    kk = st["k"]
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1][:, :kk], want[1][:, :kk])
+    assert torch.equal(got[2], want[2]) and torch.equal(got[3], want[3])
