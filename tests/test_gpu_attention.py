@@ -88,7 +88,7 @@ def test_split_kv_arrays_equal_records(hs, port, mapped):
 
 
 def test_chunks_with_empty_unions(hs, port):
-    # Every query head selects only ids below 1000 of 4096, so most 128-id
+    # Every query head selects only ids below 1000 of 4096, so most
     # chunks have an empty union for every KV head: those chunks read no row
     # and contribute nothing (and a head whose ids are all in one chunk still
     # gets its output from that chunk alone).
@@ -176,10 +176,19 @@ def test_closed_forms(hs, port, form, case):
     assert np.allclose(got, ref, rtol=TOL, atol=1e-5)
 
 
+def shuffled(hs, pool, v_words, g):
+    """The rows of a pool of 4096 B records behind a row map, and as K and V
+    arrays: (rows, records, V rows)."""
+    perm = g.permutation(len(pool)).astype(np.int32)
+    records = pool[np.argsort(perm)]  # row perm[id] holds id
+    return to_dev(perm), to_dev(records.reshape(-1)), to_dev(np.ascontiguousarray(records[:, v_words:]).reshape(-1))
+
+
 @pytest.mark.parametrize("n", [128 * 64, 128 * 64 + 1, 28671, 28672, 128 * 256 + 1, 65536])
 def test_merge_batches_and_streamed_rows(hs, port, n):
-    # the record merge reads 4, 16 or 32 chunks per thread (64, 256 and 512
-    # chunks of 128 ids), and the V rows are streamed from 28672 tokens on
+    # the record merge reads 4, 16 or 32 chunks per thread (256 chunks of 32
+    # ids, 129 of 64, 224, 257 and 512 of 128), and the V rows are streamed
+    # from 28672 tokens on; behind a row map the same bits
     g = rng(50 + n)
     k = f16_bits(g.standard_normal((n, 8, 128)))
     v = f16_bits(g.standard_normal((n, 8, 128)))
@@ -190,13 +199,17 @@ def test_merge_batches_and_streamed_rows(hs, port, n):
                                   to_dev(member_words(ids, n).reshape(-1)))
     ref = port.attention(q, pool.view(np.uint8), ids)
     assert rel_err(out.cpu().numpy().astype(np.float64), ref) <= TOL
+    rows, mapped, _ = shuffled(hs, pool, 1024, g)
+    again = hs.ops.sparse_attention(torch.from_numpy(q).cuda(), mapped, n, to_dev(member_words(ids, n).reshape(-1)),
+                                    rows=rows)
+    assert torch.equal(again, out)
 
 
 @pytest.mark.parametrize("n", [1, 31, 32, 33, 65, 8191, 8192, 8193, 16384, 16385])
 def test_chunk_lengths(hs, port, n):
     # chunks of 32 ids up to 8192 tokens, 64 up to 16384, 128 beyond: full
     # and ragged last chunks with almost every row selected, K and V rows
-    # and V rows with the scoring pass's dots
+    # and V rows with the scoring pass's dots, each also behind a row map
     g = rng(40 + n)
     k = f16_bits(g.standard_normal((n, 8, 128)))
     v = f16_bits(g.standard_normal((n, 8, 128)))
@@ -205,12 +218,30 @@ def test_chunk_lengths(hs, port, n):
     ids = [np.flatnonzero((g.random(n) < 0.95) | (np.arange(n) == n - 1)) for _ in range(32)]
     member = to_dev(member_words(ids, n).reshape(-1))
     qd = torch.from_numpy(q).cuda()
+    rows, mapped, mapped_v = shuffled(hs, pool, 1024, g)
     out = hs.ops.sparse_attention(qd, to_dev(pool.reshape(-1)), n, member)
     ref = port.attention(q, pool.view(np.uint8), ids)
     assert rel_err(out.cpu().numpy().astype(np.float64), ref) <= TOL
+    assert torch.equal(hs.ops.sparse_attention(qd, mapped, n, member, rows=rows), out)
     _, dots = hs.ops.score_logits(to_dev(f16_bits(q).reshape(-1)), qd, to_dev(k.reshape(-1)), n)
     out = hs.ops.sparse_attention_logits(dots, to_dev(v.reshape(-1)), n, member)
     assert rel_err(out.cpu().numpy().astype(np.float64), ref) <= TOL
+    assert torch.equal(hs.ops.sparse_attention_logits(dots, mapped_v, n, member, rows=rows), out)
+
+
+@pytest.mark.parametrize("n,row_bytes", [(8192, 1 << 19), (16384, 1 << 18), (16385, 1 << 18)])
+def test_v_rows_past_4_gib(hs, n, row_bytes):
+    # V rows spread over 4 GiB take the 64-bit row addressing instead of the
+    # buffer reads, in chunks of 32, 64 and 128 ids: the same bits as packed rows
+    g = rng(n)
+    v = torch.from_numpy(f16_bits(g.standard_normal((n, 1024))).view(np.int16)).cuda()
+    dots = torch.from_numpy(g.standard_normal((32, n)).astype(np.float32)).cuda()
+    ids = [np.unique(np.append(g.choice(n, size=n // 20, replace=False), n - 1)) for _ in range(32)]
+    member = to_dev(member_words(ids, n).reshape(-1))
+    want = hs.ops.sparse_attention_logits(dots, v, n, member)
+    wide = torch.empty((n, row_bytes // 2), dtype=torch.int16, device="cuda")
+    wide[:, :1024] = v
+    assert torch.equal(hs.ops.sparse_attention_logits(dots, wide, n, member, row_bytes=row_bytes), want)
 
 
 def test_workspace_of_longer_sequences_serves_shorter(hs):

@@ -61,11 +61,17 @@ def test_batched_select_matches_single_calls(hs, id_order, use_partial):
         assert torch.equal(member, m1)
 
 
-def test_batched_select_mixed_sizes_and_cover(hs):
-    # one job beyond the per-head limit: the batch runs job by job
+@pytest.mark.parametrize("longer", [None, 70000])
+def test_batched_select_mixed_sizes_and_cover(hs, longer):
+    # one launch for all jobs up to 65536 ids; with one job beyond them the
+    # batch runs job by job
     ns = [4096, 40000, 12288]
     jobs = make_jobs(hs, ns, 3000)
     outs = [hs.ops.score(j["q16"], j["keys"], j["tokens"]) for j in jobs]
+    if longer:
+        ns.insert(1, longer)
+        outs.insert(1, (torch.randn((32, longer), generator=torch.Generator(device="cuda").manual_seed(longer),
+                                    device="cuda") * 11.0).half())
     for cover in (False, True):
         res = hs.ops.select_batched([dict(scores=o, n=n) for o, n in zip(outs, ns)], 32, 2.0,
                                     0.2, scale_raw=True, cover=cover)

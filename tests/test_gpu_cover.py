@@ -42,7 +42,7 @@ def check(hs, port, raw, heads, stride, position, alpha, fp32=False):
 
 
 @pytest.mark.parametrize("heads,position", [(32, 63), (32, 1000), (8, 4095), (32, 32767),
-                                            (4, 40000)])
+                                            (4, 40000), (3, 70001)])
 @pytest.mark.parametrize("alpha", [0.5, 2.0, 1000.0])
 def test_matches_oracle(hs, port, heads, position, alpha):
     g = rng(position + int(alpha * 10))

@@ -5,8 +5,9 @@ the query and that token's K row, then selects over all n columns.
 
 Bar: bit-exact against the same selection over one-shot scores of all n
 columns (scores, ids, counts, k, tied heads, status), and against the
-oracle; per-head path, slice path, without the scorer's tile maxima, the
-current token as the new head-0 maximum, and inside select-then-score."""
+oracle; per-head launch with one and with two words per thread, slice
+launches, without the scorer's tile maxima, the current token as the new
+head-0 maximum, and inside select-then-score."""
 import ctypes
 
 import numpy as np
@@ -77,6 +78,30 @@ def test_history_plus_current_equals_one_shot(hs, port, n, peak, id_order):
     assert np.array_equal(from_dev(got[1])[:, :kk], ref_ids)
     if peak:  # the current token moved the head-0 maximum
         assert got[3]["head0_max_key"] == port.order_key(int(raw[0, n - 1]))
+
+
+@pytest.mark.parametrize("n,ratio,id_order", [(40000, 0.35, False), (65537, 0.2, False), (65537, 0.2, True)])
+@pytest.mark.parametrize("with_partial", [True, False])
+def test_slice_launches_complete_the_current_token(hs, port, n, ratio, id_order, with_partial):
+    # past 65536 columns, or with a cap too large for the rank-order sort, the
+    # slice launches follow the count that completes column n - 1
+    q, k = _inputs(n, 800 + n, peak=True)
+    qd, kd = to_dev(q.reshape(-1)), to_dev(k.reshape(-1))
+    raw = torch.full((32, n), float("nan"), dtype=torch.float16, device="cuda")
+    part = torch.empty((n - 1 + 63) // 64, dtype=torch.int32, device="cuda")
+    hs.ops.score(qd, kd, n - 1, out=raw, score_stride=n, head0_partial=part)
+    job = dict(scores=raw, n=n, current_q=qd, current_key=to_dev(k[n - 1].reshape(-1)))
+    if with_partial:
+        job["head0_partial"] = part
+    (ids, counts, _, status), = hs.ops.select_batched([job], 32, 12.0, ratio, scale_raw=True, id_order=id_order)
+    want = port.score(q, k.reshape(-1), n)
+    assert np.array_equal(from_dev(raw), want)
+    rc, kk, pids, pcounts, tied = port.select(port.scale(want), 32, n, n, 12.0, ratio)
+    st = hs.ops.read_status(status)
+    assert rc == st["code"] == 0 and st["k"] == kk > 0 and st["boundary_tied_heads"] == tied
+    assert st["head0_max_key"] == port.order_key(int(want[0, n - 1]))
+    assert np.array_equal(from_dev(counts), pcounts)
+    assert np.array_equal(from_dev(ids)[:, :kk], np.sort(pids, axis=1) if id_order else pids)
 
 
 def test_without_tile_maxima(hs):

@@ -46,7 +46,9 @@ def test_scores_and_dots(hs, n, mapped):
 
 
 @pytest.mark.parametrize("n,frac,mapped", [(4096, 0.2, False), (32768, 0.2, False),
-                                           (5000, 0.14, True), (257, 0.5, False)])
+                                           (5000, 0.14, True), (257, 0.5, False),
+                                           # (row maps over 64- and 128-id chunks)
+                                           (12001, 0.14, True), (20000, 0.14, True)])
 def test_attention_from_dots(hs, port, n, frac, mapped):
     g = rng(620 + n)
     k = rope_keys(n, 621 + n)
@@ -88,7 +90,7 @@ def test_attention_from_dots(hs, port, n, frac, mapped):
 def test_streamed_keys(hs, n):
     # keys are streamed from 36864 tokens in the dots' launch and from 65536
     # in plain scoring (single and batched): the same bits as calls below
-    # those lines over parts of the keys
+    # those lines over parts of the keys, and behind a row map
     keys = torch.empty(n * 1024, dtype=torch.float16, device="cuda")
     hs.ops.fill_rope_keys(keys, n, 1024, 8, seed=n)
     q16 = torch.empty(4096, dtype=torch.float16, device="cuda")
@@ -96,6 +98,13 @@ def test_streamed_keys(hs, n):
     q32 = torch.randn((32, 128), device="cuda")
     raw, dots = hs.ops.score_logits(q16, q32, keys, n)
     plain = hs.ops.score(q16, keys, n)
+    perm = torch.randperm(n, generator=torch.Generator(device="cuda").manual_seed(n), device="cuda")
+    shuffled = torch.empty_like(keys).view(n, 1024)
+    shuffled[perm] = keys.view(n, 1024)  # row perm[t] holds token t
+    rows, shuffled = perm.int(), shuffled.view(-1)
+    mapped, mapped_dots = hs.ops.score_logits(q16, q32, shuffled, n, rows=rows)
+    assert torch.equal(mapped, raw) and torch.equal(mapped_dots, dots)
+    assert torch.equal(hs.ops.score(q16, shuffled, n, rows=rows), plain)
     batch = hs.ops.score_batched([dict(q16=q16, keys=keys[a * 1024:], tokens=min(16384, n - a))
                                   for a in range(0, n, 16384)])
     for a, got in zip(range(0, n, 16384), batch):

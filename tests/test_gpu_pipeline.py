@@ -102,7 +102,8 @@ def test_batched_select_then_batched_score(hs, id_order):
 
 
 def test_select_then_score_off_the_per_head_path(hs):
-    # n > 32768 takes the slice launch chain: the call runs the two in turn
+    # n > 32768 takes two words per thread and no shared launch: the call runs
+    # the two in turn
     n = 40000
     layer_a, layer_b = make_jobs(hs, [n, 4096], 7300)
     raw_a = scored_layer(hs, layer_a)
@@ -118,6 +119,23 @@ def test_select_then_score_off_the_per_head_path(hs):
     torch.cuda.synchronize()
     assert torch.equal(out_b.view(torch.int16), want_b.view(torch.int16))
     assert torch.equal(part_b, want_part_b)
+    assert_select_equal(hs, job, want)
+
+
+def test_select_then_score_slice_launches(hs):
+    # past 65536 ids the slice launches, then the scoring
+    n = 70000
+    layer_b, = make_jobs(hs, [4096], 7310)
+    raw = (torch.randn((32, n), generator=torch.Generator(device="cuda").manual_seed(n), device="cuda") * 11.0).half()
+    want_b = scored_layer(hs, dict(layer_b))
+    want = expected_select(hs, select_job(hs, raw, n, None), False)
+    job = select_job(hs, raw, n, None)
+    out_b = torch.empty((32, 4096), dtype=torch.float16, device="cuda")
+    hs.ops.select_then_score([job], [dict(q16=layer_b["q16"], keys=layer_b["keys"], tokens=4096, out=out_b)],
+                             32, ALPHA, RATIO, scale_raw=True)
+    torch.cuda.synchronize()
+    assert torch.equal(out_b.view(torch.int16), want_b.view(torch.int16))
+    assert want[3]["code"] == 0 and want[3]["k"] > 0
     assert_select_equal(hs, job, want)
 
 
@@ -158,8 +176,8 @@ def kv_layers(hs, n, count, seed):
 
 @pytest.mark.parametrize("n", [32768, 3000, 40000])
 def test_pipelined_layers_equal_one_layer_at_a_time(hs, n):
-    # (n = 40000 takes the slice launch chain: the counted selection skips
-    # only the count launch there too)
+    # (n = 40000: two words per thread, selections and scorings in turn; the
+    # counted selection skips only the count launch there too)
     # score 0; per layer: select l (counted after the first) beside score l+1,
     # then attention l beside the count of l+1; the last layer alone
     layers = kv_layers(hs, n, 3, 7500 + n)
@@ -238,6 +256,36 @@ def test_counted_selection_equals_plain(hs, id_order):
     assert torch.equal(out, want_out)
     for j, w in zip(jobs, wants):
         assert_select_equal(hs, j, w)
+
+
+@pytest.mark.parametrize("n,ratio,id_order", [(40000, 0.35, False), (70000, 0.2, False), (70000, 0.2, True)])
+def test_counted_slice_launches_equal_plain(hs, n, ratio, id_order):
+    # a counted selection by the slice launches (past 65536 ids, or a cap too
+    # large for the rank-order sort) equals the same selection made at once
+    raw = (torch.randn((32, n), generator=torch.Generator(device="cuda").manual_seed(n), device="cuda") * 11.0).half()
+    cap = math.floor(n * float(np.float32(ratio)))
+    words = (n + 31) // 32
+    ids, counts, member, st = hs.ops.select(raw, 32, n, n, ALPHA, ratio, scale_raw=True, id_order=id_order,
+                                            member=torch.zeros((32, words), dtype=torch.int32, device="cuda"))
+    want = hs.ops.read_status(st)
+    assert want["code"] == 0 and want["k"] > 0
+    job = dict(scores=raw, n=n, ids=torch.full((32, cap), -1, dtype=torch.int32, device="cuda"),
+               counts=torch.full((32,), -1, dtype=torch.int32, device="cuda"),
+               member=torch.full((32, words), -1, dtype=torch.int32, device="cuda"),
+               status=hs.ops.new_status("cuda"), ws=hs.ops.workspace(hs.ops.select_workspace_bytes(32, n), "cuda"))
+    m = 4096
+    L = kv_layers(hs, m, 1, 7990)[0]
+    every = torch.full((32, m // 32), -1, dtype=torch.int32, device="cuda")
+    want_out = hs.ops.sparse_attention(L["q32"], L["k"], m, every, v_pool=L["v"], row_bytes=2048)
+    out = torch.empty((32, 128), device="cuda")
+    aws = hs.ops.workspace(hs.ops.attention_workspace_bytes(m), "cuda")
+    hs.ops.prepare_attention_then_count(L["q32"], L["k"], m, every, [job], 32, ALPHA, ratio, out=out, ws=aws,
+                                        v_pool=L["v"], row_bytes=2048, scale_raw=True, id_order=id_order)()
+    hs.ops.select(raw, 32, n, n, ALPHA, ratio, scale_raw=True, id_order=id_order, counted=True, ids=job["ids"],
+                  counts=job["counts"], member=job["member"], status=job["status"], ws=job["ws"])
+    torch.cuda.synchronize()
+    assert torch.equal(out, want_out)
+    assert_select_equal(hs, job, (ids, counts, member, want))
 
 
 def test_select_then_score_history_cover(hs):

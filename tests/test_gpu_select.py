@@ -306,11 +306,11 @@ def test_repeated_calls_share_workspace(hs, port):
             assert np.array_equal(from_dev(dev_counts), counts)
 
 
-@pytest.mark.parametrize("n", [1000, 40000])
+@pytest.mark.parametrize("n", [1000, 40000, 70001])
 def test_failed_selection_clears_member(hs, n):
     # A failed selection leaves no stale bitmaps behind for an attention that
     # follows on the stream: the member words it was given are cleared
-    # (per-head path and slice path).
+    # (per-head launch with one and with two words per thread, slice launches).
     g = rng(22)
     s = f16_bits(g.standard_normal((32, n)))
     s[0, n // 2] = 0x7E00  # NaN in head 0: nonfinite head-0 score
@@ -325,9 +325,9 @@ def test_failed_selection_clears_member(hs, n):
 
 
 def test_random_sweep_against_oracle(hs, port):
-    # seeded shapes and parameters across both launch paths: heads 1..128,
-    # n up to 40000 (the slice chain past 32768), strides with padding,
-    # quantized scores (ties) or Gaussian ones, FP32 counts on and off
+    # seeded shapes and parameters: heads 1..128, n up to 40000 (past 32768 two
+    # words per thread, or the slice launches at ratio 0.5 and 1), strides with
+    # padding, quantized scores (ties) or Gaussian ones, FP32 counts on and off
     g = rng(9091)
     for case in range(12):
         heads = int(g.choice([1, 3, 8, 32, 100, 128]))
@@ -345,6 +345,30 @@ def test_random_sweep_against_oracle(hs, port):
             vals = g.standard_normal((heads, n)) * 3.0
         s[:, :n] = f16_bits(vals)
         check_against_port(hs, port, s, heads, stride, n, alpha, ratio, fp32)
+
+
+def test_slice_launch_sweep_against_oracle(hs, port):
+    # the slice launches (65537 ids and more): any stride and alignment,
+    # raw scores scaled on the way or not, ties and Gaussian scores
+    g = rng(9093)
+    for case in range(12):
+        heads, n = int(g.choice([1, 2, 5])), int(g.integers(65537, 131073))
+        stride = n + int(g.integers(0, 20))
+        alpha, ratio = float(g.choice([0.5, 2.0, 5.0])), float(np.float32(g.choice([0.02, 0.2, 0.6])))
+        scale, offset = bool(case % 2), int(g.integers(0, 8))
+        vals = (g.integers(0, 64, size=(heads, n)) - 32) / 4.0 if case % 3 == 0 else g.standard_normal((heads, n)) * 3.0
+        s = np.full((heads, stride), hb(-60000), dtype=np.uint16)
+        s[:, :n] = f16_bits(vals * (11.0 if scale else 1.0))
+        rc, k, ids, counts, tied = port.select(port.scale(s) if scale else s, heads, stride, n, alpha, ratio, True)
+        flat = np.concatenate([np.full(offset, hb(60000), dtype=np.uint16), s.reshape(-1)[: (heads - 1) * stride + n]])
+        dev = to_dev(flat)[offset:]
+        for id_order in (False, True):
+            got, gcounts, _, status = hs.ops.select(dev, heads, stride, n, alpha, ratio, id_order=id_order,
+                                                    scale_raw=scale, fp32_counts=True)
+            st = hs.ops.read_status(status)
+            assert st["code"] == rc == 0 and st["k"] == k and st["boundary_tied_heads"] == tied, case
+            assert np.array_equal(from_dev(gcounts), counts)
+            assert np.array_equal(from_dev(got)[:, :k], np.sort(ids, axis=1) if id_order else ids), case
 
 
 def test_per_head_sweep_against_oracle(hs, port):
@@ -497,19 +521,25 @@ def test_id_order_around_the_stage(hs, port, n, k):
 @pytest.mark.parametrize("offset", range(8))
 def test_rows_off_sixteen_bytes(hs, port, offset):
     # score rows at every offset within 16 bytes (an odd stride, a base off by
-    # 0..7 ids): the count reads two aligned words per 8 ids and moves them
-    # down; the first and last ids of the scores are read one by one
+    # 0..7 ids): the count, and past 65536 ids the plan and slice launches,
+    # read two aligned words per 8 ids and move them down; the first and last
+    # ids of the scores are read one by one
     g = rng(60 + offset)
-    for n, stride in ((8, 9), (4097, 4099), (9001, 9003)):
+    for n, stride in ((8, 9), (4097, 4099), (9001, 9003), (65543, 65545)):
         s = f16_bits(g.standard_normal((8, stride)) * 3.0)
         s[0, 0] = s[7, n - 1] = hb(11.0)  # both ends are selected
         flat = np.concatenate([np.full(offset, hb(60000), dtype=np.uint16), s.reshape(-1)[: 7 * stride + n]])
-        rc, k, ids, counts, tied = port.select(s, 8, stride, n, 4.0, 0.5)
         dev = to_dev(flat)[offset:]
         assert dev.data_ptr() % 16 == 2 * offset
-        for id_order in (False, True):
-            got, gcounts, _, status = hs.ops.select(dev, 8, stride, n, 4.0, 0.5, id_order=id_order)
-            st = hs.ops.read_status(status)
-            assert st["code"] == rc == 0 and st["k"] == k and st["boundary_tied_heads"] == tied
-            assert np.array_equal(from_dev(gcounts), counts)
-            assert np.array_equal(from_dev(got)[:, :k], np.sort(ids, axis=1) if id_order else ids)
+        for scale in (False, True):
+            # (scaled scores are 11 times smaller: the same share within alpha / 11)
+            alpha = 0.375 if scale else 4.0
+            rc, k, ids, counts, tied = port.select(port.scale(s) if scale else s, 8, stride, n, alpha, 0.5)
+            assert rc == 0
+            for id_order in (False, True):
+                got, gcounts, _, status = hs.ops.select(dev, 8, stride, n, alpha, 0.5, id_order=id_order,
+                                                        scale_raw=scale)
+                st = hs.ops.read_status(status)
+                assert st["code"] == rc and st["k"] == k and st["boundary_tied_heads"] == tied
+                assert np.array_equal(from_dev(gcounts), counts)
+                assert np.array_equal(from_dev(got)[:, :k], np.sort(ids, axis=1) if id_order else ids)
