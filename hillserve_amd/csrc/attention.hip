@@ -99,10 +99,9 @@ __device__ __forceinline__ void accumulate_pair(float (&o)[4][8], const half2v (
 //  4. the chunk's exact maximum per head, p = exp(s - m) and l = sum p (no
 //     running maximum), then o += p * V as the rows land, and the record.
 // kStream: the V rows, which nothing reads again, are read with the
-// nontemporal hint, so that they leave the K rows (scored shortly before) in
-// the caches.  Eight pipelined layers of 32768 tokens take
-// 364.7 us against 368.0; no difference at 24576 and below, where the V rows
-// of a pass may come from the caches themselves.
+// nontemporal hint (so that, as the times suggest, the MALL keeps the K rows
+// scored shortly before).  Eight pipelined layers of 32768 tokens take
+// 364.7 us against 368.0; no difference at 24576 and below.
 constexpr uint32_t kStreamTokens = 28672;
 template <bool kRows, bool kStream, uint32_t kChunk>
 __global__ void __launch_bounds__(kThreads)

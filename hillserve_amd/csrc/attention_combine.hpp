@@ -20,6 +20,12 @@ namespace hs {
 // everywhere, one layer (V rows only) of 3001 / 8192 / 16384 23.0 / 26.4 /
 // 32.7 against 24.9 / 28.0 / 33.8.  More workgroups than CUs do not pay: 32 ids
 // at 16384 tokens 35.2 us, 64 at 32768 45.1 against 43.8, twice the records.
+// The softmax weights are rounded to F16 against their chunk's maximum, so a
+// shorter chunk is also nearer 64 bits: 1.3e-4 with 32 ids, 1.5e-4 with 64,
+// 1.65e-4 with 128.  What it costs is the merge: the V-only call alone with 2 %
+// of the ids selected takes 9.7 us against 8.5 at 8192 tokens (9.9 / 9.1 at
+// 16384), with 20 % 10.2 against 10.9.  (256 CUs are the whole GPU's; the
+// workspace sizes follow the chunks, so they do not depend on the device.)
 constexpr uint32_t kAttnChunk = 128;
 constexpr uint32_t kAttnShort = 256 * 32, kAttnMiddle = 256 * 64;
 inline uint32_t attn_chunk(uint32_t n) { return n <= kAttnShort ? 32u : n <= kAttnMiddle ? 64u : kAttnChunk; }

@@ -195,15 +195,15 @@ __device__ __forceinline__ const uint8_t* fallback_row(const PoolSource& ps, con
 // 195.1, 227.6 / 238.9; one workspace 16.0 / 16.4, 19.3 / 18.9, 21.5 / 21.8.
 // Bound by HBM: at 6560 slots the pack moves 269 MB (161 MB written), the
 // gather 215 MB (107 MB written).  The packed V and mask leave through
-// streaming stores, K through the caches: with all three in the caches the
-// output pushes out the pool rows that the four query heads of a KV head read
-// again, with all three streamed a workspace reused from layer to layer no
-// longer stays in the MALL.  us, all cached / all streamed / as here: 6560
+// streaming stores, K through the caches, because the times say so; the bytes
+// behind the L2 are the same with V and mask stored through the caches too
+// (pack 51.5 and 51.6 thousand KiB fetched), so what it changes lies in the
+// MALL, which has no counter.  us, all cached / all streamed / as here: 6560
 // slots, three workspaces in turn: pack with its union 68.2 / 59.8 / 59.6,
 // gather 45.9 / 43.5 / 41.6; one workspace over 30 pools: pack 49.6 / 52.1 /
-// 48.3, gather 37.9 / 41.4 / 37.9; a 64-query pack of 1664 slots with its union
-// 17.9 / 17.6 / 16.7.  (Streaming loads of the rows lose their reuse: pack with
-// its union 76.3, gather 44.5.)
+// 48.3, gather 37.9 / 41.4 / 37.9 (there the gather gains nothing); a 64-query
+// pack of 1664 slots with its union 17.9 / 17.6 / 16.7.  (With streaming loads
+// of the rows too: pack with its union 76.3, gather 44.5.)
 constexpr uint32_t kShortSlots = 256 * 8 / 32 * 64, kLineSlots = 2560;
 inline uint32_t pack_slots(uint32_t count) {
     return count <= kShortSlots && (count < kLineSlots || count % 64 != 0) ? 32u : 64u;

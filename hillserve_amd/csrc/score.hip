@@ -40,10 +40,9 @@ namespace {
 
 constexpr uint32_t kWavesPerBlock = 2;
 
-// Keys are streamed past the caches (nontemporal loads) where nothing will
-// read them again while the 256 MB MALL still holds them: they then stop
-// displacing the scores and dots that the next launches read, and a long
-// stream runs faster.  The dots' launch leaves the attention only V
+// Keys are read with the nontemporal hint where nothing will read them again
+// while the 256 MB MALL could still hold them.  The lines rest on times alone
+// (the MALL has no counter).  The dots' launch leaves the attention only V
 // rows to read, so its keys are done with: streamed from 72 MiB (36864
 // tokens).  One layer, ten pools in turn: 70.9 -> 68.7 us at 65536 tokens, 62.2
 // -> 61.7 at 40960, but 47.3 -> 47.5 at 32768 (44.8 -> 45.4 with 30 pools), where
@@ -52,8 +51,12 @@ constexpr uint32_t kWavesPerBlock = 2;
 // before (24576 tokens 39.5 -> 41.3).  A plain scoring launch is followed
 // by an attention that reads the selected K rows, so its line is 128 MiB,
 // more than the MALL keeps until then: 16 sequences of 8192 to 32768 tokens
-// 173.8 -> 155.8 us, a 65536-token cover 67.9 -> 64.3 us, while the pipelined
-// 32768-token layers (64 MiB a launch) would lose 2.4 us each.
+// 173.8 -> 155.8 us, a 65536-token cover 67.9 -> 64.3 us, three pools of 65536
+// tokens scored in turn 80.0 -> 74.6 us (105.6 -> 99.9 in 4096 B records),
+// while the pipelined 32768-token layers (64 MiB a launch) would lose 2.4 us
+// each.  Only one pool of 65536 tokens scored again and again, with nothing
+// read between, loses what the MALL would keep of it (23.3 -> 24.9 us, 31.6 in
+// records).
 constexpr uint64_t kStreamKeyBytes = uint64_t(128) << 20;
 constexpr uint64_t kStreamLogitKeyBytes = uint64_t(72) << 20;
 
@@ -81,11 +84,11 @@ score_logits_kernel(const ScoreJobs jobs, const int32_t* __restrict__ rows, uint
         gridDim.x * kWavesPerBlock, lds[w], lo, qstage[w]);
 }
 
-// Up to kShortIds (token tile, KV head) pairs, four per CU: a wave of its own
-// workgroup for each, spread over all CUs (in two-wave workgroups half the CUs
-// would hold two waves): 16 pools scored in turn 104.1 -> 95.4 us at 8192
-// tokens, 69.4 -> 66.4 at 1024, a layer of 8192 29.2 -> 24.1 with the launch
-// after it.  From 12288 tokens on the waves fill the CUs and it is slower
+// Up to kShortIds (token tile, KV head) pairs, four per CU of the whole GPU's
+// 256: a wave of its own workgroup for each, spread over all CUs (in two-wave
+// workgroups half the CUs would hold two waves): 16 pools scored in turn 104.1
+// -> 95.4 us at 8192 tokens, 69.4 -> 66.4 at 1024, a layer of 8192 29.2 -> 24.1
+// with the launch after it.  From 12288 tokens on the waves fill the CUs and it is slower
 // (30.8 -> 31.5 us a layer).
 constexpr uint32_t kShortIds = 1024;
 // Both halves of a wave's tile are in flight at once (the second otherwise
