@@ -54,7 +54,8 @@ int build_score_jobs(const hs_score_job_t* jobs, uint32_t count, ScoreJobs& out)
 // of LDS.  Waves never wait on one another.  A tile's second half is
 // requested once its first is parked in LDS, into the same registers.
 // (Both halves requested together cost 32 more VGPRs and measured slower
-// wherever the chip is full; kOneTile does it below that.)
+// wherever the chip is full; kOneTile does it for the launches of score.hip
+// that gain by it.)
 // kLogits: the same pass also produces the attention's q.k dots of the
 // tile's 64 tokens for the 4 query heads (F32 queries lo.qf), on MFMA from
 // the K values the ordered chains already hold: v_mfma_f32_4x4x4_16b_f16
