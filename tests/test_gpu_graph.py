@@ -19,7 +19,7 @@ KMAX = min(N, math.floor(N * float(np.float32(RATIO))))
 
 
 def fill_layer(hs, k, v, q16, q32, seed):
-    hs.ops.fill_rope_keys(k, N, 1024, 8, seed=seed, theta=500000.0)
+    hs.ops.fill_rope_keys(k, k.numel() // 1024, 1024, 8, seed=seed, theta=500000.0)
     hs.ops.fill_gaussian(v, seed=seed + 1)
     hs.ops.fill_gaussian(q16, seed=seed + 2)
     q32.copy_(torch.randn(q32.shape, generator=torch.Generator(device="cuda").manual_seed(seed),
@@ -34,22 +34,25 @@ def capture(fn, stream):
     return graph
 
 
-def test_decode_layer_graph_replays_equal_eager(hs):
+@pytest.mark.parametrize("n", [N, 12289])
+def test_decode_layer_graph_replays_equal_eager(hs, n):
+    # one launch of count and selection up to 8192 tokens, two beyond
+    kmax = min(n, math.floor(n * float(np.float32(RATIO))))
     dev = "cuda"
-    k = torch.empty(N * 1024, dtype=torch.float16, device=dev)
+    k = torch.empty(n * 1024, dtype=torch.float16, device=dev)
     v = torch.empty_like(k)
     q16 = torch.empty(4096, dtype=torch.float16, device=dev)
     q32 = torch.empty((32, 128), dtype=torch.float32, device=dev)
-    scores = torch.empty((32, N), dtype=torch.float16, device=dev)
-    ids = torch.empty((32, KMAX), dtype=torch.int32, device=dev)
+    scores = torch.empty((32, n), dtype=torch.float16, device=dev)
+    ids = torch.empty((32, kmax), dtype=torch.int32, device=dev)
     counts = torch.empty(32, dtype=torch.int32, device=dev)
     out = torch.empty((32, 128), dtype=torch.float32, device=dev)
     status = hs.ops.new_status(dev)
-    ws = hs.ops.workspace(hs.ops.decode_layer_workspace_bytes(N), dev)
+    ws = hs.ops.workspace(hs.ops.decode_layer_workspace_bytes(n), dev)
     outputs = (scores, ids, counts, out, status)
 
     def layer():
-        hs.ops.decode_layer(q16, q32, k, N, ALPHA, RATIO, scores=scores, ids=ids, ids_stride=KMAX,
+        hs.ops.decode_layer(q16, q32, k, n, ALPHA, RATIO, scores=scores, ids=ids, ids_stride=kmax,
                             counts=counts, out=out, status=status, ws=ws, v_pool=v, row_bytes=2048)
 
     side = torch.cuda.Stream()
@@ -68,7 +71,7 @@ def test_decode_layer_graph_replays_equal_eager(hs):
             layer()
             torch.cuda.synchronize()
             st = hs.ops.read_status(status)
-            assert st["code"] == 0 and st["k"] == KMAX, (seed, st)
+            assert st["code"] == 0 and st["k"] == kmax, (seed, st)
             for name, a, b in zip(("scores", "ids", "counts", "out", "status"), replayed, outputs):
                 assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), (seed, name)
 
